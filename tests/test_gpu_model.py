@@ -377,6 +377,26 @@ def test_chunk_tiles_beyond_fp16_take_the_rows(tmp_path, monkeypatch):
     assert np.array_equal(got["tiles"], got["rows"])
 
 
+@pytest.mark.parametrize("count", [65, 128, 129, 256, 257, 2047, 2100])
+@pytest.mark.parametrize("name", ["q8_0-d64", "q8_0-d64-g16"])
+def test_prompt_passes_match_small_passes(tmp_path, name, count):
+    # the tiled products of a prompt pass (above 64 vectors; above 256 in the
+    # wider tile; a second pass after 2,048 tokens) against passes of 64, whose
+    # products stream the weights: the same f32 sums of the same fp16 halves in
+    # another order, so within a few rounding steps of sums over 1,024 columns
+    spec = gf.LlamaSpec(**{**CHUNK_SPECS[name], "context": 2200, "layers": 2})
+    path = spec.write(tmp_path / "m.gguf")
+    tokens = [int(t) for t in np.random.default_rng(count).integers(0, spec.vocab, count)]
+    mine = native.NativeModel(path, max_blocks=2 * (2200 // 16) + 8, block_tokens=16)
+    got = mine.prefill(mine.new_sequence(), tokens)
+    small = mine.new_sequence()
+    for lo in range(0, count, 64):
+        want = mine.prefill(small, tokens[lo:lo + 64])
+    ok, err = close(got, want)
+    say(name, count, "relative logit difference", err)
+    assert ok, err
+
+
 def test_prefill_matches_reference_last_logits(tmp_path, ref_capi):
     # tvara_sequence_prefill: the last token's logits of a chunked pass, with
     # decode_batch's checks, messages and rollback

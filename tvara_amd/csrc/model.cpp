@@ -257,20 +257,22 @@ void DeviceModel::matvec(const Weight& w, const float* v, const MatvecSegment* s
     launch_matvec(static_cast<const float*>(w.f32.ptr), w.rows, w.cols, v, seg, nseg, s);
 }
 
-void DeviceModel::ensure_batch(size_t n) {
-    if (n <= batch_cap_) return;
+void DeviceModel::ensure_batch(size_t n, size_t logits) {
+    if (n <= batch_cap_ && logits <= logits_cap_) return;
+    n = std::max(n, batch_cap_);
+    logits = std::max(logits, logits_cap_);
     const ModelConfig& c = cfg_;
     const size_t H = c.hidden, I = c.intermediate, KV = c.kv_width(), L = c.layers, F = sizeof(float);
-    if (!part_rows_) {
-        auto note = [&](const Weight& w) { part_rows_ = std::max(part_rows_, static_cast<size_t>(batch_splits_max(w)) * w.rows); };
-        for (const Layer& l : layers_) {
-            note(l.qkv);
-            note(l.out);
-            note(l.gate_up);
-            note(l.down);
-        }
-        note(has_output_ ? output_ : embedding_);
+    size_t part = 0;
+    auto note = [&](const Weight& w) { part = std::max(part, batch_part_floats(w, static_cast<int>(n))); };
+    for (const Layer& l : layers_) {
+        note(l.qkv);
+        note(l.out);
+        note(l.gate_up);
+        note(l.down);
     }
+    // unsplit logits are written in place
+    part = std::max(part, batch_part_floats(has_output_ ? output_ : embedding_, static_cast<int>(logits)));
     bx_.ensure(n * H * F);
     bnorm_.ensure(n * H * F);
     bq_.ensure(n * H * F);
@@ -280,13 +282,14 @@ void DeviceModel::ensure_batch(size_t n) {
     bvapp_.ensure(n * L * KV * F);
     battn_.ensure(n * H * F);
     bgate_.ensure(n * I * F);
-    blogits_.ensure(n * c.vocab * F);
     brope_.ensure(n * c.head_dim() * F);
     btok_.ensure(n * sizeof(uint32_t));
-    bpart_.ensure(n * part_rows_ * F);
+    bpart_.ensure(part * F);
+    blogits_.ensure(logits * c.vocab * F);
     bhalves_.ensure((n + 15) / 16 * 16 * std::max(H, I) * 2 * sizeof(_Float16));
     bunscale_.ensure(n * F);
     batch_cap_ = n;
+    logits_cap_ = logits;
 }
 
 void DeviceModel::StepEvents::ensure() {
@@ -331,7 +334,7 @@ void DeviceModel::decode_many(const uint64_t* sequences, const uint32_t* tokens,
         }
         return;
     }
-    ensure_batch(n);
+    ensure_batch(n, n);
     hipStream_t s = cache_->stream();
     const int N = static_cast<int>(n), KV = static_cast<int>(c.kv_width());
     stage_rows(tokens, positions.data(), n);
@@ -504,19 +507,19 @@ void DeviceModel::decode_chunk(uint64_t sequence, const uint32_t* tokens, size_t
         }
         return;
     }
-    const size_t rows = std::min(n, kChunkRows);
-    if (rows > static_cast<size_t>(std::numeric_limits<int>::max() / std::max<size_t>(c.vocab, c.hidden)))
-        throw std::invalid_argument("decode batch too large");
-    ensure_batch(rows);
-    hipStream_t s = cache_->stream();
-    const int heads = static_cast<int>(c.heads);
-    std::vector<size_t> positions(rows);
-    std::vector<uint64_t> seq_of_row(rows, sequence);
     // TVARA_CHUNK_ATTENTION=rows (read on every call) keeps the f32 rows, the
     // reference's arithmetic, for every layout
     const char* choice = std::getenv("TVARA_CHUNK_ATTENTION");
     const bool rows_only = choice && std::strcmp(choice, "rows") == 0;
     const bool tiles = !rows_only && prefill_x3_supported(cache_->layout(), 1);
+    const size_t rows = std::min(n, last_only && tiles ? kPromptRows : kChunkRows);
+    if (rows > static_cast<size_t>(std::numeric_limits<int>::max() / std::max<size_t>(c.vocab, c.hidden)))
+        throw std::invalid_argument("decode batch too large");
+    ensure_batch(rows, last_only ? 1 : rows);
+    hipStream_t s = cache_->stream();
+    const int heads = static_cast<int>(c.heads);
+    std::vector<size_t> positions(rows);
+    std::vector<uint64_t> seq_of_row(rows, sequence);
     for (size_t c0 = 0; c0 < n; c0 += rows) {
         const size_t m = std::min(rows, n - c0);
         positions.resize(m);

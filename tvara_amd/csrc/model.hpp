@@ -65,8 +65,9 @@ void launch_matvec_q8(const Weight& w, const float* v, const MatvecSegment* seg,
 // epilogue below writes them, with a power-of-two unscale per vector), f32
 // weights read x [n][cols].
 int batch_splits(const Weight& w, int n);
-// the most splits any n gives (the size of a partial-sum buffer)
-int batch_splits_max(const Weight& w);
+// the most floats that a product of up to n vectors writes (the size of a
+// partial-sum buffer)
+size_t batch_part_floats(const Weight& w, int n);
 void launch_batch_product(const Weight& w, const float* x, const _Float16* halves, const float* unscale, int n,
                           float* out, hipStream_t s);
 // the rows of row tiles [tile0, tile1) of an unsplit Q8_0 product (out as for
@@ -125,7 +126,7 @@ public:
     // independent decode() calls; on failure no sequence changes
     void decode_many(const uint64_t* sequences, const uint32_t* tokens, size_t n, float* logits_host);
     // n consecutive tokens at the end of `sequence` in one pass per chunk of
-    // up to kChunkRows tokens (the batched products, each layer's K/V written
+    // up to kChunkRows or kPromptRows tokens (the batched products, each layer's K/V written
     // into the cache, then the rows' causal attention over it): the logits of
     // n decode() calls, of every token or, with last_only, of the last one
     // only.  The attention runs as MFMA tiles with every f32 operand split
@@ -136,7 +137,13 @@ public:
     // again on the rows.  On failure the sequence may hold part of the
     // tokens; the caller truncates it.
     void decode_chunk(uint64_t sequence, const uint32_t* tokens, size_t n, float* logits_host, bool last_only);
-    static constexpr size_t kChunkRows = 512;
+    // A prompt's passes hold up to kPromptRows tokens: a quarter of the launches
+    // and products of 2,048 vectors, at which the tiled GEMM runs at 1.1 times
+    // its rate at 512 (a 2,048-token prompt on Llama-3.2-1B: 24.9 ms in passes
+    // of 512 on the kernels of that time, 13.5 in one pass on the tiled GEMM).
+    // Calls that return every token's logits keep kChunkRows, for the size of
+    // the logits buffer, and so do passes on the f32 rows, for their partials.
+    static constexpr size_t kChunkRows = 512, kPromptRows = 2048;
 
 private:
     struct Layer {
@@ -164,7 +171,6 @@ private:
     // batch work buffers, grown to the largest batch seen
     DeviceBuffer bx_, bnorm_, bq_, bk_, bv_, bkapp_, bvapp_, battn_, bgate_, blogits_, brope_, btok_, bpart_, bhalves_,
         bunscale_;
-    size_t part_rows_ = 0;  // largest splits x rows of a batched product
     PinnedBuffer bhost_;
     HostCopier copier_;
     // the batched step's synchronisation: an event after the last layer's
@@ -182,8 +188,9 @@ private:
         ~StepEvents();
     };
     StepEvents step_events_;
-    size_t batch_cap_ = 0;
-    void ensure_batch(size_t n);
+    size_t batch_cap_ = 0, logits_cap_ = 0;
+    // work buffers for n rows, of which `logits` rows give logits
+    void ensure_batch(size_t n, size_t logits);
     // the widths the batched products and epilogues take
     bool batched_widths() const;
     // tokens and each row's (cos, sin) to the device, then the rows'

@@ -852,167 +852,180 @@ __global__ __launch_bounds__(256) void batch_q8_kernel(const Q8BatchArgs a) {
     }
 }
 
-// Weight-stationary form of the same product, for any number of vectors in
-// one launch.  A workgroup of four waves owns RT row tiles over one K split
-// of a.groups_per_split groups (a multiple of four): it first converts the
-// split's int8 weights and scales into LDS, eight loads a thread requested
-// before the first conversion, and then each wave multiplies them against
-// its vector tiles in turn (tiles w, w + 4, ...), UG groups a step, the
-// activation halves of the next step (the next tile's first, at a tile's
-// end) in flight while a step is summed.  No barrier follows the staging.
-// The arithmetic per group is the chunked kernel's, so the sums are the
-// same.  LDS: groups_per_split * RT KiB of fp16 weights, then the scales.
-template <int RT, int UG>
-__global__ __launch_bounds__(256) void batch_q8_ws_kernel(const Q8BatchArgs a) {
-    extern __shared__ half8 wsh[];  // [groups_per_split][RT][64], then scales [RT][pairs][16] dwords
-    const int gps = a.groups_per_split, pps = gps / 2;
-    uint32_t* wsd = reinterpret_cast<uint32_t*>(wsh + static_cast<size_t>(gps) * RT * 64);
+// The same product as a tiled GEMM, for many vectors.  A workgroup of eight
+// waves (two by four) owns 2*VT vector tiles by sixteen row tiles over one K
+// split, a wave VT by four of them, so that the operands a wave reads from LDS
+// per group, (2*VT + 4) KiB, feed 8*VT MFMAs.  K advances a group pair a step,
+// two steps ahead of the products: the activation halves go from memory
+// straight into one of three LDS buffers (16 bytes a lane, in the operand
+// order they are stored in), the int8 weights into one of two register sets
+// and from there, converted once for the workgroup, into one of two LDS
+// buffers; the scales a lane needs stay in registers.  A step has one barrier.
+// With VT = 4 the buffers take all 160 KB of LDS: one workgroup a CU, two
+// waves a SIMD.
+// Workgroups are numbered so that each XCD takes a contiguous run of tiles
+// (eight row blocks by the vector blocks), whose operands its L2 then shares.
+// Only even group counts come here (no pair is half dead).  Row tiles past the
+// matrix read zeros; vector tiles past the batch read the last tile again and
+// are not stored.
+//
+// Bound: issue on the SIMDs.  At 2,048 vectors of the 16,384 x 2,048 gate|up
+// MFMAs take 43% of the cycles and the vector instructions (two thirds of them
+// the four scale FMAs a product) 32-43%, and the two add up rather than
+// overlap; LDS is busy 22%, without a bank conflict.
+// MI355X, 3,072 / 2,048 / 16,384 x 2,048 and 2,048 x 8,192, against the kernel
+// it replaced (weights kept in LDS, activations read through L1 by every
+// wave), which took four times its time at 512: 78.6 / 45.3 / 330 / 161 us at
+// 2,048 vectors against 137 / 112 / 530 / 264 (834 TFLOP/s of fp16 products on
+// the third), and 28.5 / 25.9 / 89 / 45 us at 512 against 34 / 28 / 133 / 66.
+template <int VT>
+__global__ __launch_bounds__(512, 2) void batch_q8_pipe_kernel(const Q8BatchArgs a) {
+    constexpr int BV = 2 * VT, BR = 16;  // vector and row tiles of a workgroup
+    constexpr int XL = BV * 4 / 8;       // KiB of halves a wave loads per pair
+    // separate arrays, so that the compiler sees that a step's reads do not
+    // touch the buffers in flight and does not wait for them
+    __shared__ u32x4 x0[BV][4][64], x1[BV][4][64], x2[BV][4][64];  // [vector tile][group * 2 + part][lane]
+    __shared__ half8 w0[2][BR][64], w1[2][BR][64];                 // [group][row tile][lane]
     const int tid = static_cast<int>(threadIdx.x), lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int gbeg = static_cast<int>(blockIdx.y) * gps;
-    const int gend = min(a.groups, gbeg + gps);
-    const int pbeg = gbeg / 2;
-    // every slot of the split's share is staged, the pairs past its end too
-    // (the next split's bytes, or zeros past the view): each weight and
-    // scale a dead group meets is finite, so its zero activations add zero
-    const int np = pps;
-    const int t0 = a.tile0 + static_cast<int>(blockIdx.x) * RT;
-    const int tiles_here = min(RT, a.tiles - t0);
+    const int vh = wave & 1, rh = wave >> 1;
+    // logical tile of this workgroup
+    const int nrb = (a.tiles - a.tile0 + BR - 1) / BR, nvb = (a.n_total_tiles + BV - 1) / BV;
+    int vb, rb;
+    {
+        const int total = nrb * nvb, b = static_cast<int>(blockIdx.x);
+        const int per = total / 8, extra = total % 8, xcd = b % 8;
+        const int id = xcd * per + min(xcd, extra) + b / 8;
+        const int band = id / (8 * nvb), rows_here = min(8, nrb - band * 8), in = id - band * 8 * nvb;
+        vb = in / rows_here;
+        rb = band * 8 + in - vb * rows_here;
+    }
+    const int t0 = a.tile0 + rb * BR;
+    const int tiles_here = min(BR, a.tiles - t0);
+    const int pbeg = static_cast<int>(blockIdx.y) * (a.groups_per_split / 2);
+    const int np = min(a.pairs, pbeg + a.groups_per_split / 2) - pbeg;
     const __amdgpu_buffer_rsrc_t qv =
         view(a.q + static_cast<size_t>(t0) * a.pairs * 64, static_cast<uint32_t>(tiles_here * a.pairs) * 1024u);
     const __amdgpu_buffer_rsrc_t dv = view(reinterpret_cast<const uint32_t*>(a.d) + static_cast<size_t>(t0) * a.pairs * 16,
                                            static_cast<uint32_t>(tiles_here * a.pairs) * 64u);
-    // ---- staging: RT x np pairs x 64 lanes of int8, eight loads a thread a round
-    {
-        constexpr int B = 8;
-        const int units = RT * np * 64;
-        for (int e0 = tid; e0 < units; e0 += 256 * B) {
-            uint4 raw[B];
-#pragma unroll
-            for (int i = 0; i < B; ++i) {
-                const int e = e0 + 256 * i;  // past `units`: a read past the view (zeros), not stored
-                const int l = e & 63, rp = e >> 6, r = rp / np, p = rp - r * np;
-                raw[i] = __builtin_bit_cast(
-                    uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                               qv, static_cast<uint32_t>(((r * a.pairs + p) * 64 + l) * 16), pbeg * 1024, 0));
-            }
-#pragma unroll
-            for (int i = 0; i < B; ++i) {
-                const int e = e0 + 256 * i;
-                if (e >= units) break;
-                const int l = e & 63, rp = e >> 6, r = rp / np, p = rp - r * np;
-                wsh[((2 * p) * RT + r) * 64 + l] = i8x8_to_half8(make_uint2(raw[i].x, raw[i].y));
-                wsh[((2 * p + 1) * RT + r) * 64 + l] = i8x8_to_half8(make_uint2(raw[i].z, raw[i].w));
-            }
-        }
-        const int dunits = RT * np * 16;
-        for (int e = tid; e < dunits; e += 256) {
-            const int row = e & 15, rp = e >> 4, r = rp / np, p = rp - r * np;
-            wsd[(r * pps + p) * 16 + row] = __builtin_amdgcn_raw_buffer_load_b32(
-                dv, static_cast<uint32_t>(((r * a.pairs + p) * 16 + row) * 4), pbeg * 64, 0);
-        }
-    }
-    __syncthreads();
-
-    // ---- products: this wave's vector tiles (w, w + 4, ...), UG groups a
-    // unit, one stream of (tile, unit) steps double-buffered across tiles
-    const int ntv = (a.n + 15) / 16;
-    const uint32_t xbytes = static_cast<uint32_t>(a.n_total_tiles) * static_cast<uint32_t>(a.groups) * 2048u;
-    const __amdgpu_buffer_rsrc_t xv = view(a.halves, xbytes);
+    const __amdgpu_buffer_rsrc_t xv =
+        view(a.halves, static_cast<uint32_t>(a.n_total_tiles) * static_cast<uint32_t>(a.groups) * 2048u);
     const uint32_t xoff = static_cast<uint32_t>(lane) * 16u;
-    const int nunits = (gend - gbeg + UG - 1) / UG;
-    const int mytiles = wave < ntv ? (ntv - 1 - wave) / 4 + 1 : 0;
-    const int steps = mytiles * nunits;
-    auto load_x = [&](int jt, int u, u32x4 (&x)[UG][2]) {
-        const int vt = wave + 4 * jt;
+    const uint32_t qoff = static_cast<uint32_t>((wave * a.pairs * 64 + lane) * 16);  // row tiles wave, wave + 8
+    const uint32_t doff = static_cast<uint32_t>((rh * 4 * a.pairs * 16 + (lane & 15)) * 4);
+
+    uint4 ra[2], rb2[2];
+    uint32_t da[4], db[4], dc[4];
+    auto load_w = [&](int p, uint4 (&raw)[2], uint32_t (&dn)[4]) {
 #pragma unroll
-        for (int c = 0; c < UG; ++c) {
-            const int g = gbeg + UG * u + c;
-            const int so = g < gend ? ((a.vt0 + vt) * a.groups + g) * 2048 : static_cast<int>(xbytes);
-            x[c][0] = __builtin_amdgcn_raw_buffer_load_b128(xv, xoff, so, 0);
-            x[c][1] = __builtin_amdgcn_raw_buffer_load_b128(xv, xoff + 1024u, so, 0);
+        for (int i = 0; i < 2; ++i)
+            raw[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                   qv, qoff, ((8 * i * a.pairs) + pbeg + p) * 1024, 0));
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            dn[r] = __builtin_amdgcn_raw_buffer_load_b32(dv, doff, (r * a.pairs + pbeg + p) * 64, 0);
+    };
+    auto load_x = [&](int p, u32x4 (&x)[BV][4][64]) {
+#pragma unroll
+        for (int i = 0; i < XL; ++i) {
+            const int t = (wave * XL + i) / 4, part = (wave * XL + i) % 4;
+            const int vt = min(vb * BV + t, a.n_total_tiles - 1);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(xv, (__attribute__((address_space(3))) void*)&x[t][part][0], 16, xoff,
+                                                     (vt * a.groups + 2 * (pbeg + p)) * 2048 + part * 1024, 0, 0);
         }
     };
-    float4v acc[RT];
+    auto stage = [&](const uint4 (&raw)[2], half8 (&ws)[2][BR][64]) {
 #pragma unroll
-    for (int r = 0; r < RT; ++r) acc[r] = float4v{0.f, 0.f, 0.f, 0.f};
-    float* out = a.out + static_cast<size_t>(blockIdx.y) * a.n_total * a.rows;
-    auto step = [&](int jt, int u, const u32x4 (&x)[UG][2]) {
-        uint32_t dd[RT][UG / 2];
+        for (int i = 0; i < 2; ++i) {
+            ws[0][wave + 8 * i][lane] = i8x8_to_half8(make_uint2(raw[i].x, raw[i].y));
+            ws[1][wave + 8 * i][lane] = i8x8_to_half8(make_uint2(raw[i].z, raw[i].w));
+        }
+    };
+    float4v acc[VT][4];
 #pragma unroll
-        for (int r = 0; r < RT; ++r)
+    for (int v = 0; v < VT; ++v)
 #pragma unroll
-            for (int p = 0; p < UG / 2; ++p)
-                dd[r][p] = wsd[(r * pps + min((UG / 2) * u + p, pps - 1)) * 16 + (lane & 15)];
+        for (int r = 0; r < 4; ++r) acc[v][r] = float4v{0.f, 0.f, 0.f, 0.f};
+    auto compute = [&](const u32x4 (&x)[BV][4][64], const half8 (&ws)[2][BR][64], const uint32_t (&dd)[4]) {
 #pragma unroll
-        for (int c = 0; c < UG; ++c) {
-            const int gl = min(UG * u + c, gps - 1);  // a group past the split reads a staged one: its x is zero
-            const half8 xh = __builtin_bit_cast(half8, x[c][0]), xl = __builtin_bit_cast(half8, x[c][1]);
-            half8 w[RT];
+        for (int g = 0; g < 2; ++g) {
+            half8 w[4];
+            float d[4];
 #pragma unroll
-            for (int r = 0; r < RT; ++r) w[r] = wsh[(gl * RT + r) * 64 + lane];
-            float4v cc[RT];
+            for (int r = 0; r < 4; ++r) {
+                w[r] = ws[g][rh * 4 + r][lane];
+                d[r] = half_bits_to_float(static_cast<uint16_t>(dd[r] >> (16 * g)));
+            }
 #pragma unroll
-            for (int r = 0; r < RT; ++r)
-                cc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, w[r], float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            for (int v = 0; v < VT; ++v) {
+                const half8 xh = __builtin_bit_cast(half8, x[vh * VT + v][2 * g][lane]);
+                const half8 xl = __builtin_bit_cast(half8, x[vh * VT + v][2 * g + 1][lane]);
+                float4v cc[4];
 #pragma unroll
-            for (int r = 0; r < RT; ++r) cc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, w[r], cc[r], 0, 0, 0);
+                for (int r = 0; r < 4; ++r)
+                    cc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, w[r], float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-            for (int r = 0; r < RT; ++r) {
-                const float d = half_bits_to_float(static_cast<uint16_t>(dd[r][c / 2] >> (c % 2 ? 16 : 0)));
+                for (int r = 0; r < 4; ++r) cc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, w[r], cc[r], 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) acc[r][i] = fmaf(d, cc[r][i], acc[r][i]);
+                for (int r = 0; r < 4; ++r)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[v][r][i] = fmaf(d[r], cc[r][i], acc[v][r][i]);
             }
         }
-        if (u + 1 < nunits) return;
-        // the tile's last unit: lane l holds row l%16 of each row tile for
-        // vectors 4(l/16) + i of vector tile vt
-        const int vt = wave + 4 * jt;
+    };
+    // Step p: wait for this wave's part of pair p (requested two steps ago; the
+    // newest step's loads stay in flight) and for its LDS writes, meet the
+    // others, request pair p + 2 into the buffer read in step p - 1, multiply
+    // pair p, convert pair p + 1.  Loads past the split repeat its last pair,
+    // so that every step issues the same number and the count below holds.
+    constexpr int kPerStep = 2 + 4 + XL;
+    auto step = [&](int p, const u32x4 (&xc)[BV][4][64], u32x4 (&xn)[BV][4][64], const half8 (&wc)[2][BR][64],
+                    half8 (&wn)[2][BR][64], const uint32_t (&dcur)[4], uint32_t (&dnxt)[4], uint4 (&rload)[2],
+                    const uint4 (&rstage)[2]) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kPerStep) : "memory");
+        const int pn = min(p + 2, np - 1);
+        load_w(pn, rload, dnxt);
+        load_x(pn, xn);
+        compute(xc, wc, dcur);
+        __builtin_amdgcn_sched_barrier(0);  // the conversion waits for loads: not ahead of the products
+        stage(rstage, wn);
+    };
+    load_w(0, ra, da);
+    load_x(0, x0);
+    load_w(min(1, np - 1), rb2, db);
+    load_x(min(1, np - 1), x1);
+    stage(ra, w0);
+    for (int p = 0;; p += 6) {
+        step(p, x0, x2, w0, w1, da, dc, ra, rb2);
+        if (p + 1 >= np) break;
+        step(p + 1, x1, x0, w1, w0, db, da, rb2, ra);
+        if (p + 2 >= np) break;
+        step(p + 2, x2, x1, w0, w1, dc, db, ra, rb2);
+        if (p + 3 >= np) break;
+        step(p + 3, x0, x2, w1, w0, da, dc, rb2, ra);
+        if (p + 4 >= np) break;
+        step(p + 4, x1, x0, w0, w1, db, da, ra, rb2);
+        if (p + 5 >= np) break;
+        step(p + 5, x2, x1, w1, w0, dc, db, rb2, ra);
+        if (p + 6 >= np) break;
+    }
+    // no load may be in flight into this workgroup's LDS when it ends
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // lane l holds row l%16 of each row tile for vectors 4(l/16) + i
+    float* out = a.out + static_cast<size_t>(blockIdx.y) * a.n_total * a.rows;
+#pragma unroll
+    for (int v = 0; v < VT; ++v)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int jl = vt * 16 + 4 * (lane >> 4) + i;
-            if (jl >= a.n) continue;
-            const int j = a.vt0 * 16 + jl;
+            const int j = (vb * BV + vh * VT + v) * 16 + 4 * (lane >> 4) + i;
+            if (j >= a.n) continue;
             const float us = a.unscale[j];
 #pragma unroll
-            for (int r = 0; r < RT; ++r) {
-                const int row = (t0 + r) * 16 + (lane & 15);
-                if (t0 + r < a.tiles && row < a.rows) out[static_cast<size_t>(j) * a.rows + row] = acc[r][i] * us;
+            for (int r = 0; r < 4; ++r) {
+                const int tile = t0 + rh * 4 + r, row = tile * 16 + (lane & 15);
+                if (tile < a.tiles && row < a.rows) out[static_cast<size_t>(j) * a.rows + row] = acc[v][r][i] * us;
             }
         }
-#pragma unroll
-        for (int r = 0; r < RT; ++r) acc[r] = float4v{0.f, 0.f, 0.f, 0.f};
-    };
-    if (steps == 0) return;
-    // the (tile, unit) of the next step to load and of the step to compute,
-    // counted up rather than divided out of a flat index (8% of the
-    // product's time at 256-512 vectors went to the divisions)
-    u32x4 xa[UG][2], xb[UG][2];
-    int jn = 0, un = 0, jc = 0, uc = 0;
-    auto next_load = [&](u32x4 (&x)[UG][2]) {
-        const bool past = jn >= mytiles;
-        load_x(past ? mytiles - 1 : jn, past ? nunits - 1 : un, x);
-        if (++un == nunits) {
-            un = 0;
-            ++jn;
-        }
-    };
-    auto next_step = [&](const u32x4 (&x)[UG][2]) {
-        step(jc, uc, x);
-        if (++uc == nunits) {
-            uc = 0;
-            ++jc;
-        }
-    };
-    next_load(xa);
-    for (int k = 0;; k += 2) {
-        next_load(xb);
-        next_step(xa);
-        if (k + 1 >= steps) break;
-        next_load(xa);
-        next_step(xb);
-        if (k + 2 >= steps) break;
-    }
 }
 
 // ---------------------------------------------------------- batch epilogues
@@ -1414,45 +1427,34 @@ F32Plan f32_plan(int rows, int cols) {
     return p;
 }
 
-// Weight-stationary plan: RT row tiles per workgroup (four from 1,024 row
-// tiles up, else two) and the K split that keeps a workgroup's fp16 weights
-// within 64 KiB of LDS, split further (in steps of four groups, never below
-// eight) while the launch has fewer than 512 workgroups.
-struct WsPlan {
-    int rt, gps, gx, splits;
-    size_t lds;
+// Plan of the tiled GEMM: VT = 4 (128 vectors a workgroup) above 256 vectors,
+// else 2, and K split while the launch has fewer than 256 workgroups (one a
+// CU), into at most eight splits of at least eight groups.  MI355X, the four
+// products of a Llama-3.2-1B layer together: VT = 2 takes 110 us at 256
+// vectors, 173 at 384 and 200 at 512, VT = 4 129, 167 and 180.
+struct PipePlan {
+    int vt, gx, per, splits;  // vector tiles a wave, workgroups per split, groups per split, splits
 };
-WsPlan ws_plan(const Weight& w) {
-    WsPlan p{};
-    const int tiles = w.tiles(), groups = w.groups();
-    p.rt = tiles >= 1024 ? 4 : 2;
-    p.gx = (tiles + p.rt - 1) / p.rt;
-    const int cap = 64 / p.rt;  // groups of fp16 weights in 64 KiB
-    int splits = (groups + cap - 1) / cap;
-    while (p.gx * splits < 512 && (groups + splits) / (splits + 1) >= 8) ++splits;
-    p.gps = (groups + splits - 1) / splits;
-    p.gps = (p.gps + 3) / 4 * 4;
-    if (p.gps > cap) p.gps = cap / 4 * 4;
-    p.splits = (groups + p.gps - 1) / p.gps;
-    p.lds = static_cast<size_t>(p.gps) * p.rt * 1024 + static_cast<size_t>(p.rt) * (p.gps / 2) * 64;
+PipePlan pipe_plan(const Weight& w, int n, int tiles, int most_splits = 8) {
+    PipePlan p{};
+    const int vtiles = (n + 15) / 16;
+    p.vt = n > 256 ? 4 : 2;
+    p.gx = ((tiles + 15) / 16) * ((vtiles + 2 * p.vt - 1) / (2 * p.vt));
+    const int want = std::min({std::max(1, 256 / p.gx), std::max(1, w.groups() / 8), most_splits});
+    p.per = ((w.groups() + want - 1) / want + 1) / 2 * 2;  // whole pairs
+    p.splits = (w.groups() + p.per - 1) / p.per;
     return p;
 }
 
-// The weight-stationary kernel from 128 vectors (matrices under 1,024 row
-// tiles) or 256 (under 4,096); the chunked kernel otherwise.  MI355X,
-// Llama-3.2-1B shapes, weights from HBM: QKV / output / gate|up / down at 512
-// vectors 35.6 / 28.8 / 117 / 70.8 us against 59.9 / 51.0 / 138.5 / 100.6;
-// at 128 vectors 13.5 / 11.0 / 48.3 / 23.9 against 16.2 / 13.4 / 37.6 /
-// 26.8; at 64 vectors, and for the 8,016-tile logits at every size, the
-// chunked kernel is faster (gate|up 18.9 against 32.2 us at 64; logits 841
-// against 862-891 us at 512).
-bool ws_for(const Weight& w, int n) {
-    const int t = w.tiles();
-    return w.q8 && t < 4096 && (n >= 256 || (n >= 128 && t < 1024));
-}
+// The tiled GEMM above 64 vectors, where the chunked kernel needs a second
+// launch that reads the weights again (MI355X, a layer's four products: 79 us
+// against 87 at 96 vectors, 81 against 93 at 128); at 64 the chunked kernel
+// takes 45 us, this one 67.
+bool pipe_for(const Weight& w, int n) { return w.q8 && w.groups() % 2 == 0 && n > 64; }
 
-void launch_ws(const Weight& w, const WsPlan& p, int tile0, int tile1, const _Float16* halves, const float* unscale,
-               int n, float* out, hipStream_t s) {
+// row tiles [tile0, tile1), K in `per` groups a split
+void launch_pipe(const Weight& w, const PipePlan& p, int tile0, int tile1, const _Float16* halves,
+                 const float* unscale, int n, float* out, hipStream_t s) {
     Q8BatchArgs a{};
     a.q = static_cast<const uint4*>(w.q.ptr);
     a.d = static_cast<const uint16_t*>(w.d.ptr);
@@ -1464,35 +1466,37 @@ void launch_ws(const Weight& w, const WsPlan& p, int tile0, int tile1, const _Fl
     a.groups = w.groups();
     a.pairs = w.pairs();
     a.n = n;
-    a.vt0 = 0;
     a.n_total = n;
     a.n_total_tiles = (n + 15) / 16;
-    a.groups_per_split = p.gps;
+    a.groups_per_split = p.per;
     a.out = out;
     if (static_cast<double>(a.n_total_tiles) * a.groups * 2048 >= 2147483648.0)
         throw std::invalid_argument("batched product input above 2 GiB");
-    const dim3 grid((tile1 - tile0 + p.rt - 1) / p.rt, p.splits);
-    if (p.rt == 4)
-        launch("model_matvec_q8", batch_q8_ws_kernel<4, 4>, grid, dim3(256), p.lds, s, a);
+    const dim3 grid(p.gx, p.splits);
+    if (p.vt == 4)
+        launch("model_matvec_q8", batch_q8_pipe_kernel<4>, grid, dim3(512), 0, s, a);
     else
-        launch("model_matvec_q8", batch_q8_ws_kernel<2, 4>, grid, dim3(256), p.lds, s, a);
+        launch("model_matvec_q8", batch_q8_pipe_kernel<2>, grid, dim3(512), 0, s, a);
 }
 }  // namespace
 
 int batch_splits(const Weight& w, int n) {
     if (!w.q8) return f32_plan(w.rows, w.cols).splits;
-    return ws_for(w, n) ? ws_plan(w).splits : q8_plan(w).splits;
+    return pipe_for(w, n) ? pipe_plan(w, n, w.tiles()).splits : q8_plan(w).splits;
 }
 
-int batch_splits_max(const Weight& w) {
-    if (!w.q8) return f32_plan(w.rows, w.cols).splits;
-    return std::max(ws_plan(w).splits, q8_plan(w).splits);
+size_t batch_part_floats(const Weight& w, int n) {
+    // the splits depend on the count of 16-vector tiles
+    size_t most = 0;
+    for (int j = std::min(n, 16); j; j = j < n ? std::min(n, j + 16) : 0)
+        most = std::max(most, static_cast<size_t>(batch_splits(w, j)) * j * w.rows);
+    return most;
 }
 
 void launch_batch_product(const Weight& w, const float* x, const _Float16* halves, const float* unscale, int n,
                           float* out, hipStream_t s) {
-    if (ws_for(w, n)) {
-        launch_ws(w, ws_plan(w), 0, w.tiles(), halves, unscale, n, out, s);
+    if (pipe_for(w, n)) {
+        launch_pipe(w, pipe_plan(w, n, w.tiles()), 0, w.tiles(), halves, unscale, n, out, s);
     } else if (w.q8) {
         const Q8Plan p = q8_plan(w);
         for (int j0 = 0; j0 < n; j0 += 64) {
@@ -1541,8 +1545,8 @@ void launch_batch_product_tiles(const Weight& w, int tile0, int tile1, const _Fl
                                 int n, float* out, hipStream_t s) {
     if (!w.q8 || batch_splits(w, n) != 1 || tile0 < 0 || tile0 >= tile1 || tile1 > w.tiles())
         throw std::invalid_argument("row-tile range of a batched product needs an unsplit Q8_0 matrix");
-    if (ws_for(w, n)) {
-        launch_ws(w, ws_plan(w), tile0, tile1, halves, unscale, n, out, s);
+    if (pipe_for(w, n)) {
+        launch_pipe(w, pipe_plan(w, n, tile1 - tile0, 1), tile0, tile1, halves, unscale, n, out, s);
         TVARA_HIP(hipGetLastError());
         return;
     }
