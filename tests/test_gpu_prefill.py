@@ -607,3 +607,68 @@ def test_pipelined_kernel_ragged_chunks(device, oracle, monkeypatch, group, tpb)
                            for q, s, st, c in zip(qs, rs, starts, counts)])
     ok, err = bf16_ok(pipe, want, SHORT_ROWS)
     assert ok, err
+
+
+F32_TILE_SPECS = [(1510, 1000, 500), (300, 0, 300), (70, 67, 3), (1, 0, 1)]
+
+
+@pytest.mark.parametrize("fmt", ["f32", "q8_0"])
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("group,tpb", [(1, 16), (3, 64), (4, 1024), (8, 16), (12, 32)])  # 12: slices of six heads
+def test_f32_tiles(device, oracle, group, tpb, dim, fmt):
+    # a batch above the f32 tiles' threshold of work, with key splits (some of
+    # them empty for the short sequences), rows and keys that fill neither a
+    # wave nor a tile, and ten cached tokens past the chunk; rows at the chunk's
+    # ends and at tile and workgroup edges against the oracle
+    heads = 24
+    say("prefill f32 tiles group", group, "tpb", tpb, "dim", dim, fmt)
+    dev, ref, ds, rs, qs = build(device, oracle, heads, heads // group, dim, F32_TILE_SPECS, seed=90 + group, tpb=tpb,
+                                 q8=fmt == "q8_0")
+    starts = [s for _, s, _ in F32_TILE_SPECS]
+    counts = [r for _, _, r in F32_TILE_SPECS]
+    got = attention.prefill_batch(dev, np.concatenate(qs), ds, starts, counts, 0, heads, 4096, precision="f32")
+    row0 = 0
+    for q, s, st, c in zip(qs, rs, starts, counts):
+        for lo, n in [(0, 3), (22, 4), (30, 4), (126, 4), (c - 3, 3)]:
+            lo, n = max(0, min(lo, c - 1)), min(n, c)
+            n = min(n, c - lo)
+            want = ref.fused_prompt_attention(q[lo:lo + n], s, 0, st + lo, n, heads, 4096).reshape(n, -1)
+            part = got[row0 + lo:row0 + lo + n]
+            assert refmath.close(part, want, 1e-5), (lo, refmath.max_rel(part, want))
+        row0 += c
+
+
+@pytest.mark.parametrize("dim", [64, 128])
+def test_f32_tiles_non_finite(device, dim):
+    # values that are not finite reach the rows that see them and no others (a
+    # masked probability is not multiplied by them); a key that is not finite
+    # fails the call if a row sees it, and does not if none does
+    heads, kv_heads, n, start, rows = 24, 6, 1510, 1000, 500
+    w = kv_heads * dim
+    k, v = (synth.normal(3, t, n * w).reshape(n, w) for t in "kv")
+    q = synth.normal(3, "q", rows * heads * dim).reshape(rows, heads * dim)
+
+    def run(k, v):
+        c = device.PagedCache(1, kv_heads, dim, 16, n // 16 + 4, fmt=device.F32)
+        s = c.create_sequence()
+        c.append_many(s, k, v)
+        return attention.prefill_batch(c, q, [s], [start], [rows], 0, heads, 4096, precision="f32")
+
+    clean = run(k, v)
+    at = 1203
+    for bad in (np.nan, np.inf):
+        vb = v.copy()
+        vb[at, dim + 5] = bad
+        vb[n - 1] = np.nan  # past the chunk
+        got = run(k, vb).reshape(rows, heads, dim)
+        hit = np.zeros(got.shape, bool)
+        hit[at - start:, 4:8, 5] = True
+        assert np.array_equal(~np.isfinite(got), hit)
+        keep = clean.reshape(rows, heads, dim)
+        assert refmath.close(got[~hit], keep[~hit], 1e-6)
+    kb = k.copy()
+    kb[n - 1] = np.inf
+    assert np.array_equal(run(kb, v), clean)
+    kb[at, 3] = np.inf
+    with pytest.raises(ValueError, match="invalid online attention input"):
+        run(kb, v)

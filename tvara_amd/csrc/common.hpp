@@ -143,16 +143,24 @@ struct PrefillArgs {
     int layer;
     int heads, group;
     const int32_t* tables;
-    const int4* seqs;  // x: table offset, y: start, z: rows, w: first query row
+    // two entries a workgroup, by blockIdx.x (PrefillPlan::build): the
+    // sequence (x: table offset, y: start, z: rows, w: first query row), then
+    // x: KV head, y: first chunk position, z: first key tile (f32 tiles)
+    const int4* work;
+    int workgroups;  // a multiple of eight; the lists' padding has no rows
     const float* q;    // [sum rows][heads][head_dim]
     float* out;
     float qscale;
     int* err;
-    int chunk_tiles;  // query tiles per (sequence, KV head) pair (set by the launcher)
-    int pairs;        // sequences x KV heads
     // as DecodeArgs::kv_share: lay.kv_heads and group describe kv_share
     // virtual KV heads per KV head (GQA groups above eight)
     int kv_share;
+    // f32 tiles: the key tiles are cut into `splits` runs of split_tiles, whose
+    // partial outputs, [split][row][heads][head_dim], and (maximum in log2
+    // units, normaliser) pairs, [split][row][heads][2], a second kernel merges
+    int splits, split_tiles, total_rows;
+    float* part_acc;
+    float* part_ml;
 };
 
 // launchers (kernels.hip)
@@ -198,7 +206,19 @@ bool prefill_bf16_supported(const BlockLayout& lay, int group);
 // x3: the f32-accurate variant (three products per product of split
 // operands), on the blocks the bf16 tiles take
 bool prefill_x3_supported(const BlockLayout& lay, int group);
-void launch_prefill_bf16(const PrefillArgs& a, int nseqs, int max_rows, hipStream_t s, bool x3 = false);
+void launch_prefill_bf16(const PrefillArgs& a, hipStream_t s, bool x3 = false);
+int prefill_bf16_positions(int group);  // chunk positions of a workgroup
+// prefill_f32.hip: the same layouts in f32
+void launch_prefill_f32(const PrefillArgs& a, hipStream_t s);
+int prefill_f32_positions(const BlockLayout& lay, int group);
+// how the f32 tiles cover n chunks of rows[i] tokens after start[i] cached
+// ones: key splits and the tiles of each; use false where the decode kernels
+// are faster, row by row
+struct F32TileShape {
+    bool use;
+    int splits, split_tiles;
+};
+F32TileShape prefill_f32_shape(const BlockLayout& lay, int group, size_t n, const size_t* start, const size_t* rows);
 
 // kernel timing (profile.cpp)
 // Per-kernel timing for tvara_profile_*: while enabled, every launch made

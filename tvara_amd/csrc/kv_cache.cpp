@@ -716,6 +716,67 @@ void AttnPlan::check_after(hipEvent_t after) {
     finish_check();
 }
 
+// The tile kernels' workgroups.  Ids go to the eight XCDs round-robin and,
+// within an XCD, to its shader engines in turn, each id waiting for its
+// engine: ids in order of (chunk tile, sequence), many of them empty for a
+// ragged batch, left engines idle while others held the long sequences.  So
+// the list holds only workgroups with rows, in runs of equal work per XCD that
+// keep a (sequence, KV head)'s tiles together, as they share its keys in the
+// XCD's L2, and each XCD's run is ordered from the most keys to the fewest
+// (MI355X, four chunks of 200-900 tokens after 500-3,000 at head_dim 128 on
+// the three-product tiles: 439 -> 261 us; even batches unchanged).
+std::vector<int4> PrefillPlan::work_list(const std::vector<int4>& seqs, int kv_heads, int positions) const {
+    constexpr int kXcds = 8, kCus = 32, kTileKeys = 64;
+    struct Item {
+        int seq, head, q0, tile0;
+        int64_t tiles;
+    };
+    std::vector<Item> items, empty;
+    int64_t total = 0;
+    for (int i = 0; i < static_cast<int>(seqs.size()); ++i) {
+        const int start = seqs[i].y, rows = seqs[i].z;
+        for (int h = 0; h < kv_heads; ++h)
+            for (int q0 = (rows - 1) / positions * positions; q0 >= 0; q0 -= positions) {
+                const int all = (start + std::min(q0 + positions, rows) + kTileKeys - 1) / kTileKeys;
+                for (int s = 0; s < splits; ++s) {
+                    const int t0 = s * split_tiles;
+                    const int64_t t = splits == 1 ? all : std::max(0, std::min(split_tiles, all - t0));
+                    (t ? items : empty).push_back({i, h, q0, t0, t});
+                    total += t;
+                }
+            }
+    }
+    // up to four rounds of the CUs, no XCD takes more workgroups than its CUs
+    // need rounds for: one more would add a whole round (256 workgroups of
+    // 200-250 tiles, 33 of them on one XCD: 1,003 against 548 us)
+    const int64_t count = static_cast<int64_t>(items.size()), round = kXcds * kCus;
+    const int64_t cap = count <= 4 * round ? (count + round - 1) / round * kCus : count;
+    std::vector<std::vector<Item>> run(kXcds);
+    int64_t before = 0, x = 0;
+    for (int64_t i = 0; i < count; ++i) {
+        const bool full = static_cast<int64_t>(run[x].size()) == cap, share = before * kXcds >= total * (x + 1);
+        if (x + 1 < kXcds && (full || (share && count - i <= cap * (kXcds - 1 - x)))) ++x;
+        run[x].push_back(items[i]);
+        before += items[i].tiles;
+    }
+    for (auto& r : run)
+        std::stable_sort(r.begin(), r.end(), [](const Item& a, const Item& b) { return a.tiles > b.tiles; });
+    // splits without keys write that they have none
+    for (size_t i = 0; i < empty.size(); ++i) run[i % kXcds].push_back(empty[i]);
+    size_t longest = 0;
+    for (const auto& r : run) longest = std::max(longest, r.size());
+    if (longest * kXcds > static_cast<size_t>(std::numeric_limits<int>::max()))
+        throw std::invalid_argument("attention batch too large");
+    std::vector<int4> list(2 * kXcds * longest, make_int4(0, 0, 0, 0));
+    for (int r = 0; r < kXcds; ++r)
+        for (size_t k = 0; k < run[r].size(); ++k) {
+            const Item& it = run[r][k];
+            list[2 * (k * kXcds + r)] = seqs[it.seq];
+            list[2 * (k * kXcds + r) + 1] = make_int4(it.head, it.q0, it.tile0, 0);
+        }
+    return list;
+}
+
 void PrefillPlan::build(DeviceCache* c, const uint64_t* sequences, size_t n, size_t h, size_t context,
                         const size_t* start, const size_t* rows, int prec) {
     cache = c;
@@ -725,34 +786,18 @@ void PrefillPlan::build(DeviceCache* c, const uint64_t* sequences, size_t n, siz
     if (n > static_cast<size_t>(std::numeric_limits<int>::max())) throw std::invalid_argument("attention batch too large");
     heads = static_cast<int>(h);
     group = static_cast<int>(h / g.kv_heads);
-    count = static_cast<int>(n);
     precision = prec;
-    std::vector<uint64_t> seq_of_row;
-    std::vector<size_t> cached;
     total_rows = 0;
-    max_rows = 0;
     for (size_t i = 0; i < n; ++i) {
         const size_t length = c->sequence(sequences[i]).length;
         // fused_prompt_attention (attention.hpp:85-87)
         if (!rows[i] || start[i] >= length || rows[i] > length - start[i])
             throw std::invalid_argument("invalid causal prompt chunk");
         if (length > context) throw std::invalid_argument("invalid fused attention shape");
-        if (prec == 0) {
-            for (size_t j = 0; j < rows[i]; ++j) {
-                seq_of_row.push_back(sequences[i]);
-                cached.push_back(start[i] + j + 1);
-            }
-        }
         total_rows += rows[i];
-        max_rows = std::max(max_rows, static_cast<int>(std::min<size_t>(rows[i], std::numeric_limits<int>::max())));
     }
     if (total_rows > static_cast<size_t>(std::numeric_limits<int>::max()))
         throw std::invalid_argument("attention batch too large");
-    if (prec == 0) {
-        rows_plan.build(c, seq_of_row, cached, {}, heads, 0);
-        epoch = rows_plan.epoch;
-        return;
-    }
     // groups above eight: slices of at most eight query heads, each a virtual
     // KV head of the tile kernel
     kv_share = 1;
@@ -761,7 +806,31 @@ void PrefillPlan::build(DeviceCache* c, const uint64_t* sequences, size_t n, siz
         while (group % slice) --slice;
         kv_share = group / slice;
     }
-    if (!prefill_bf16_supported(c->layout(), group / kv_share))
+    const bool tiles = prefill_bf16_supported(c->layout(), group / kv_share);
+    on_rows = prec == 0;
+    splits = 1;
+    split_tiles = 0;
+    if (prec == 0 && tiles) {
+        BlockLayout lay = c->layout();
+        lay.kv_heads *= kv_share;
+        const F32TileShape f = prefill_f32_shape(lay, group / kv_share, n, start, rows);
+        on_rows = !f.use;
+        splits = f.splits;
+        split_tiles = f.split_tiles;
+    }
+    if (on_rows) {
+        std::vector<uint64_t> seq_of_row;
+        std::vector<size_t> cached;
+        for (size_t i = 0; i < n; ++i)
+            for (size_t j = 0; j < rows[i]; ++j) {
+                seq_of_row.push_back(sequences[i]);
+                cached.push_back(start[i] + j + 1);
+            }
+        rows_plan.build(c, seq_of_row, cached, {}, heads, 0);
+        epoch = rows_plan.epoch;
+        return;
+    }
+    if (!tiles)
         throw std::invalid_argument(
             "bf16 prefill needs f32 or Q8_0 blocks of 16 to 1,024 tokens (a power of two, under 2 GiB) and head_dim "
             "64 or 128");
@@ -776,11 +845,16 @@ void PrefillPlan::build(DeviceCache* c, const uint64_t* sequences, size_t n, siz
     }
     if (tab.size() > static_cast<size_t>(std::numeric_limits<int32_t>::max()))
         throw std::invalid_argument("attention batch too large");
+    const std::vector<int4> list = work_list(sq, static_cast<int>(g.kv_heads) * kv_share,
+                                             prec == 0 ? prefill_f32_positions(c->layout(), group / kv_share)
+                                                       : prefill_bf16_positions(group / kv_share));
+    workgroups = static_cast<int>(list.size() / 2);
     void* pt = tables.ensure(std::max<size_t>(tab.size() * sizeof(int32_t), 16));
-    void* ps = seqs.ensure(sq.size() * sizeof(int4));
+    void* pw = work.ensure(list.size() * sizeof(int4));
     void* pe = err.ensure(sizeof(int));
+    if (splits > 1) part.ensure(static_cast<size_t>(splits) * total_rows * heads * (g.head_dim + 2) * sizeof(float));
     TVARA_HIP(hipMemcpy(pt, tab.data(), tab.size() * sizeof(int32_t), hipMemcpyHostToDevice));
-    TVARA_HIP(hipMemcpy(ps, sq.data(), sq.size() * sizeof(int4), hipMemcpyHostToDevice));
+    TVARA_HIP(hipMemcpy(pw, list.data(), list.size() * sizeof(int4), hipMemcpyHostToDevice));
     TVARA_HIP(hipMemset(pe, 0, sizeof(int)));
     epoch = c->epoch();
 }
@@ -788,7 +862,7 @@ void PrefillPlan::build(DeviceCache* c, const uint64_t* sequences, size_t n, siz
 void PrefillPlan::launch(int layer, const float* q, float* out, hipStream_t s) {
     if (layer < 0 || static_cast<size_t>(layer) >= cache->geometry().layers)
         throw std::invalid_argument("invalid fused attention shape");
-    if (precision == 0) {
+    if (on_rows) {
         rows_plan.launch(layer, q, nullptr, nullptr, out, s);
         return;
     }
@@ -804,18 +878,29 @@ void PrefillPlan::launch(int layer, const float* q, float* out, hipStream_t s) {
     a.heads = heads;
     a.group = group / kv_share;
     a.tables = static_cast<const int32_t*>(tables.ptr);
-    a.seqs = static_cast<const int4*>(seqs.ptr);
+    a.work = static_cast<const int4*>(work.ptr);
+    a.workgroups = workgroups;
     a.q = q;
     a.out = out;
     a.qscale = static_cast<float>(1.4426950408889634 / std::sqrt(static_cast<double>(cache->geometry().head_dim)));
     a.err = pinned_err ? static_cast<int*>(flag.ptr) : static_cast<int*>(err.ptr);
-    launch_prefill_bf16(a, count, max_rows, s, precision == 2);
+    if (precision == 0) {
+        a.splits = splits;
+        a.split_tiles = split_tiles;
+        a.total_rows = static_cast<int>(total_rows);
+        a.part_acc = static_cast<float*>(part.ptr);
+        if (splits > 1)
+            a.part_ml = a.part_acc + static_cast<size_t>(splits) * total_rows * heads * cache->geometry().head_dim;
+        launch_prefill_f32(a, s);
+    } else {
+        launch_prefill_bf16(a, s, precision == 2);
+    }
     cache->leave(s);
     last_stream = s;
 }
 
 void PrefillPlan::use_pinned_error() {
-    if (precision == 0) {
+    if (on_rows) {
         rows_plan.use_pinned_error();
         return;
     }
@@ -825,7 +910,7 @@ void PrefillPlan::use_pinned_error() {
 }
 
 void PrefillPlan::check_after(hipEvent_t after) {
-    if (precision == 0) {
+    if (on_rows) {
         rows_plan.check_after(after);
         return;
     }
@@ -842,7 +927,7 @@ void PrefillPlan::check_after(hipEvent_t after) {
 }
 
 void PrefillPlan::check() {
-    if (precision == 0) {
+    if (on_rows) {
         rows_plan.check();
         return;
     }

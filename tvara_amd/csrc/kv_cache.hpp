@@ -226,11 +226,13 @@ struct AttnPlan {
 struct PrefillPlan {
     DeviceCache* cache = nullptr;
     uint64_t epoch = 0;
-    int heads = 0, group = 0, count = 0, max_rows = 0, precision = 0;
-    int kv_share = 1;  // bf16: GQA groups above eight run as slices (as AttnPlan)
+    int heads = 0, group = 0, precision = 0, workgroups = 0;
+    int kv_share = 1;  // tiles: GQA groups above eight run as slices (as AttnPlan)
+    bool on_rows = false;  // f32 through the decode kernels (rows_plan), not the tiles
     size_t total_rows = 0;
     AttnPlan rows_plan;
-    DeviceBuffer tables, seqs, err;
+    int splits = 1, split_tiles = 0;  // f32 tiles (prefill_f32_shape)
+    DeviceBuffer tables, work, err, part;
     // the tile kernels set the error flag in pinned host memory instead
     // (use_pinned_error: no copy back before a check)
     PinnedBuffer flag;
@@ -241,6 +243,8 @@ struct PrefillPlan {
     PrefillPlan& operator=(const PrefillPlan&) = delete;
     void build(DeviceCache* c, const uint64_t* sequences, size_t count, size_t heads, size_t context,
                const size_t* start, const size_t* rows, int precision);
+    // two entries a workgroup of the tile kernels (PrefillArgs::work)
+    std::vector<int4> work_list(const std::vector<int4>& seqs, int kv_heads, int positions) const;
     void use_pinned_error();
     void launch(int layer, const float* q, float* out, hipStream_t s);
     void check();

@@ -37,7 +37,7 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
 constexpr float kThreshold = 8.0f;
-constexpr int kRows = 32, kKeys = 64;
+constexpr int kRows = 32, kKeys = 64, kWavesPerGroup = 8;
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
@@ -100,23 +100,10 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_bf16_kernel(const Prefill
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int g = lane >> 4, r16 = lane & 15;
-    // XCD-aware order: workgroups are dispatched to the 8 XCDs round-robin by
-    // id, so the chunk tiles of one (sequence, KV head) pair get ids of one
-    // residue mod 8 and share that XCD's L2 for their common K/V tiles.
-    // Within an XCD the ids run from the last chunk tile to the first (the
-    // most keys to the fewest), pairs fastest: the dispatcher hands the next
-    // id to the first CU that frees up, so the heaviest tiles start first and
-    // the lightest fill in behind them (measured: 111.6 against 114.5 us on
-    // the 8 x (2,048 + 512) chunk).
-    const int id = static_cast<int>(blockIdx.x), xcd = id & 7, k = id >> 3;
-    const int groups8 = (a.pairs + 7) >> 3;
-    const int pair = (k % groups8) * 8 + xcd, ct = a.chunk_tiles - 1 - k / groups8;
-    if (pair >= a.pairs) return;
-    const int kh = pair % a.lay.kv_heads;
-    const int4 sd = a.seqs[pair / a.lay.kv_heads];  // table offset, start, rows, first query row
-    const int start = sd.y, nrows = sd.z;
-    const int q0 = ct * QT;
-    if (q0 >= nrows) return;  // the whole workgroup: chunk_tiles covers the longest chunk
+    // the plan's work list (heaviest first within each XCD)
+    const int4 sd = a.work[2 * blockIdx.x], wk = a.work[2 * blockIdx.x + 1];
+    const int start = sd.y, nrows = sd.z, kh = wk.x, q0 = wk.y;
+    if (!nrows) return;  // the list's padding
     const int kmax = start + min(q0 + QT, nrows);  // keys this workgroup reads: [0, kmax)
     const int ntiles = (kmax + kKeys - 1) / kKeys;
     const int pw0 = q0 + wave * PW;
@@ -563,15 +550,9 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_pipe_kernel(const Prefill
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, r16 = lane & 15;
     // workgroup order as in prefill_bf16_kernel
-    const int id = static_cast<int>(blockIdx.x), xcd = id & 7, k = id >> 3;
-    const int groups8 = (a.pairs + 7) >> 3;
-    const int pair = (k % groups8) * 8 + xcd, ct = a.chunk_tiles - 1 - k / groups8;
-    if (pair >= a.pairs) return;
-    const int kh = pair % a.lay.kv_heads;
-    const int4 sd = a.seqs[pair / a.lay.kv_heads];
-    const int start = sd.y, nrows = sd.z;
-    const int q0 = ct * QT;
-    if (q0 >= nrows) return;
+    const int4 sd = a.work[2 * blockIdx.x], wk = a.work[2 * blockIdx.x + 1];
+    const int start = sd.y, nrows = sd.z, kh = wk.x, q0 = wk.y;
+    if (!nrows) return;  // the list's padding
     const int kmax = start + min(q0 + QT, nrows);
     const int ntiles = (kmax + kKeys - 1) / kKeys;
     const int pw0 = q0 + wave * PW;
@@ -893,16 +874,12 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_pipe_kernel(const Prefill
 // x3 (three products per product) always takes the plain kernel, over f32
 // or Q8_0 blocks (d * q dequantised when staged, then split).
 template <int D, int G, int TPB>
-void launch_gt(const PrefillArgs& a, int nseqs, int max_rows, bool x3, hipStream_t s) {
+void launch_gt(const PrefillArgs& b, bool x3, hipStream_t s) {
     const char* env = std::getenv("TVARA_PREFILL_PIPE");
     const bool pipe = env ? std::atoi(env) != 0 : D == 64;
-    const bool q8 = a.lay.format == kQ8;
-    constexpr int W = 8, QT = W * (kRows / G);  // chunk positions per workgroup
-    PrefillArgs b = a;
-    b.chunk_tiles = (max_rows + QT - 1) / QT;
-    b.pairs = nseqs * a.lay.kv_heads;
-    const int groups8 = (b.pairs + 7) / 8;  // ids = 8 XCDs x chunk tiles x pair groups
-    const dim3 grid(8 * groups8 * b.chunk_tiles), block(64 * W);
+    const bool q8 = b.lay.format == kQ8;
+    constexpr int W = kWavesPerGroup;
+    const dim3 grid(b.workgroups), block(64 * W);
     if (x3) {
         if (q8)
             launch("paged_prefill_x3", prefill_bf16_kernel<D, G, W, true, TPB, true>, grid, block, 0, s, b);
@@ -923,13 +900,13 @@ void launch_gt(const PrefillArgs& a, int nseqs, int max_rows, bool x3, hipStream
 // blocks of 16 tokens fold the block arithmetic at compile time; other
 // powers of two read it from the layout
 template <int G>
-void launch_g(const PrefillArgs& a, int nseqs, int max_rows, bool x3, hipStream_t s) {
+void launch_g(const PrefillArgs& a, bool x3, hipStream_t s) {
     if (a.lay.head_dim == 128)
-        a.lay.tpb == 16 ? launch_gt<128, G, 16>(a, nseqs, max_rows, x3, s)
-                        : launch_gt<128, G, 0>(a, nseqs, max_rows, x3, s);
+        a.lay.tpb == 16 ? launch_gt<128, G, 16>(a, x3, s)
+                        : launch_gt<128, G, 0>(a, x3, s);
     else
-        a.lay.tpb == 16 ? launch_gt<64, G, 16>(a, nseqs, max_rows, x3, s)
-                        : launch_gt<64, G, 0>(a, nseqs, max_rows, x3, s);
+        a.lay.tpb == 16 ? launch_gt<64, G, 16>(a, x3, s)
+                        : launch_gt<64, G, 0>(a, x3, s);
 }
 
 }  // namespace
@@ -943,21 +920,23 @@ bool prefill_bf16_supported(const BlockLayout& lay, int group) {
 
 bool prefill_x3_supported(const BlockLayout& lay, int group) { return prefill_bf16_supported(lay, group); }
 
-void launch_prefill_bf16(const PrefillArgs& a, int nseqs, int max_rows, hipStream_t s, bool x3) {
+int prefill_bf16_positions(int group) { return kWavesPerGroup * (kRows / group); }
+
+void launch_prefill_bf16(const PrefillArgs& a, hipStream_t s, bool x3) {
     if (!prefill_bf16_supported(a.lay, a.group))
         throw std::invalid_argument(
             "bf16 prefill needs f32 or Q8_0 blocks of 16 to 1,024 tokens (a power of two, under 2 GiB), "
             "head_dim 64 or 128, and a GQA slice of 1-8 heads");
-    if (nseqs <= 0 || max_rows <= 0) return;
+    if (a.workgroups <= 0) return;
     switch (a.group) {
-        case 1: launch_g<1>(a, nseqs, max_rows, x3, s); break;
-        case 2: launch_g<2>(a, nseqs, max_rows, x3, s); break;
-        case 3: launch_g<3>(a, nseqs, max_rows, x3, s); break;
-        case 4: launch_g<4>(a, nseqs, max_rows, x3, s); break;
-        case 5: launch_g<5>(a, nseqs, max_rows, x3, s); break;
-        case 6: launch_g<6>(a, nseqs, max_rows, x3, s); break;
-        case 7: launch_g<7>(a, nseqs, max_rows, x3, s); break;
-        default: launch_g<8>(a, nseqs, max_rows, x3, s); break;
+        case 1: launch_g<1>(a, x3, s); break;
+        case 2: launch_g<2>(a, x3, s); break;
+        case 3: launch_g<3>(a, x3, s); break;
+        case 4: launch_g<4>(a, x3, s); break;
+        case 5: launch_g<5>(a, x3, s); break;
+        case 6: launch_g<6>(a, x3, s); break;
+        case 7: launch_g<7>(a, x3, s); break;
+        default: launch_g<8>(a, x3, s); break;
     }
     TVARA_HIP(hipGetLastError());
 }
