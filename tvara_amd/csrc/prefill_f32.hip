@@ -21,15 +21,20 @@
 // Sums.  A score is D/16 chains of four steps, summed pairwise; 32 keys'
 // contribution to the output is a chain of eight steps from zero, added to the
 // running output: chains as short as the decode kernels', where one over all
-// keys would round more the longer the context (relative 2-norm error against
-// 64 bits on the ragged chunk below: XX against YY of the decode kernels).  Softmax in log2 units with the lazy rescale of the decode
+// keys would round more the longer the context (relative error in the 2-norm
+// against 64 bits, six chunks of 33-700 tokens after 300-1,600, decode kernels
+// then tiles: 3.8e-7 and 3.1e-7 at 32 x 8 heads of 64, 3.6e-7 and 3.1e-7 of
+// 128).  Softmax in log2 units with the lazy rescale of the decode
 // kernels.  A score that is not finite sets *err (OnlineAttention::update's
 // rejection, attention.hpp:11), whether or not it would have mattered.
 //
-// Bound: the f32 matrix rate (157 TFLOP/s), an eighth of what the bf16 split
-// products would take but with nothing rounded below f32.
+// Bound: the f32 matrix rate (157 TFLOP/s), plus the softmax's vector work,
+// which adds to it.  MI355X, against the same rows through the decode kernels
+// (which read every key once per row from L2 and multiply on the vector ALU):
+// those six chunks 715 -> 328 us (87 TFLOP/s) and 1,337 -> 641 us; 8 x 512 after
+// 2,000 tokens 2,610 -> 735 us (103 TFLOP/s); 400 rows of four sequences after
+// 2,000 over Q8_0 blocks 470 -> 328 us.
 #include <algorithm>
-#include <cstdlib>
 
 #include "common.hpp"
 #include "device_util.hpp"
@@ -416,8 +421,19 @@ int prefill_f32_positions(const BlockLayout& lay, int group) {
     return lay.head_dim == 128 ? 8 * (16 / group) : 4 * (32 / group);
 }
 
+// Tiles or rows: a launch of tiles costs 10-12 us before its first result and
+// runs at 45-105 TFLOP/s, the decode kernels cost 5 and run at 20-40 (f32) or
+// 33-60 (Q8_0).  MI355X, tiles against rows: 25 against 26 us at 0.54 GFLOP,
+// 32 against 31.5 at 0.66, 31 against 44 at 1.0, 34 against 58 at 1.1; over
+// Q8_0 blocks 70 against 72 at 3.2 and 61 against 74 at 4.2.
+//
+// Key splits: one workgroup per CU where the chunk alone gives fewer (64 rows
+// after 4,000 tokens, head_dim 64: 40 us in 256 units of work, 44 in 512;
+// 256 rows after 1,000 at 128: 72, 89, 103 in 1,024), and units of a quarter of
+// a CU's share up to 1,024 workgroups, where whole rounds of unequal
+// workgroups leave a tail (six chunks of 33-700 tokens: 328 us against 431
+// unsplit).  At least two tiles a split.
 F32TileShape prefill_f32_shape(const BlockLayout& lay, int group, size_t n, const size_t* start, const size_t* rows) {
-    const char* e = std::getenv("TP_F32");
     const size_t qt = prefill_f32_positions(lay, group);
     size_t wgs = 0, work = 0, longest = 0;
     double pairs = 0;  // (query, key) pairs
@@ -432,13 +448,12 @@ F32TileShape prefill_f32_shape(const BlockLayout& lay, int group, size_t n, cons
     wgs *= lay.kv_heads;
     const double flops = 4.0 * lay.kv_heads * group * lay.head_dim * pairs;
     F32TileShape f{};
-    f.use = e ? atoi(e) : flops >= (lay.format == kQ8 ? 3e9 : 0.7e9);
+    f.use = flops >= (lay.format == kQ8 ? 3e9 : 0.7e9);
     f.splits = 1;
     f.split_tiles = static_cast<int>(longest);
     if (wgs < 1024) {
-        const char* es = std::getenv("TP_SLOTS");
-        const size_t slots = es ? atoi(es) : wgs < 256 ? 256 : 1024;
-        const size_t per = std::max<size_t>(2, (work + slots - 1) / slots);
+        const size_t units = wgs < 256 ? 256 : 1024;
+        const size_t per = std::max<size_t>(2, (work + units - 1) / units);
         f.split_tiles = static_cast<int>(std::min(per, longest));
         f.splits = static_cast<int>((longest + f.split_tiles - 1) / f.split_tiles);
     }
