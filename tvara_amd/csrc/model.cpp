@@ -416,7 +416,7 @@ void DeviceModel::layer_stack(size_t n, const Attend& attend) {
     // what follows its product (RoPE; the residual add with the next
     // RMSNorm; SwiGLU) and writes the next product's input.
     launch_resid_norm(nullptr, 0, x, at(layers_[0].attn_norm, 0), N, H, c.rms_epsilon, rows_for(layers_[0].qkv, norm),
-                      halves_for(layers_[0].qkv), unscale, s);
+                      halves_for(layers_[0].qkv), unscale, halves_by_line(layers_[0].qkv, N), s);
     for (size_t l = 0; l < c.layers; ++l) {
         Layer& L = layers_[l];
         float* kl = at(bk_, l * n * c.kv_width());
@@ -426,20 +426,21 @@ void DeviceModel::layer_stack(size_t n, const Attend& attend) {
                             c.interleaved_rope, at(brope_, 0), q, kl, vl, s);
         attend(static_cast<int>(l), q, kl, vl, attn);
         if (l + 1 == c.layers) TVARA_HIP(hipEventRecord(step_events_.attn, s));
-        if (L.out.q8) launch_split_halves(attn, N, H, halves, unscale, s);
+        if (L.out.q8) launch_split_halves(attn, N, H, halves, unscale, halves_by_line(L.out, N), s);
         launch_batch_product(L.out, attn, halves, unscale, N, part, s);
         launch_resid_norm(part, batch_splits(L.out, N), x, at(L.ffn_norm, 0), N, H, c.rms_epsilon,
-                          rows_for(L.gate_up, norm), halves_for(L.gate_up), unscale, s);
+                          rows_for(L.gate_up, norm), halves_for(L.gate_up), unscale, halves_by_line(L.gate_up, N), s);
         launch_batch_product(L.gate_up, norm, halves, unscale, N, part, s);
         launch_swiglu_epilogue(part, batch_splits(L.gate_up, N), N, I, rows_for(L.down, gate), halves_for(L.down), unscale,
-                               s, L.gate_up.interleaved);
+                               halves_by_line(L.down, N), s, L.gate_up.interleaved);
         launch_batch_product(L.down, gate, halves, unscale, N, part, s);
         // after the last layer the rows stay too: the logits of chosen rows
         // are taken from them
         const bool last = l + 1 == c.layers;
+        const Weight& next = last ? logits_w : layers_[l + 1].qkv;
         launch_resid_norm(part, batch_splits(L.down, N), x, last ? at(final_norm_, 0) : at(layers_[l + 1].attn_norm, 0), N,
-                          H, c.rms_epsilon, last ? norm : rows_for(layers_[l + 1].qkv, norm),
-                          halves_for(last ? logits_w : layers_[l + 1].qkv), unscale, s);
+                          H, c.rms_epsilon, last ? norm : rows_for(next, norm), halves_for(next), unscale,
+                          halves_by_line(next, N), s);
     }
 }
 
@@ -452,7 +453,8 @@ DeviceModel::LogitsBands DeviceModel::launch_logits(size_t n, size_t row0) {
     auto* halves = static_cast<_Float16*>(bhalves_.ptr);
     float* unscale = at(bunscale_, 0);
     // rows after the first of the final norm: their halves again, from vector 0
-    if (row0 && logits_w.q8) launch_split_halves(norm, N, static_cast<int>(c.hidden), halves, unscale, s);
+    if (row0 && logits_w.q8) launch_split_halves(norm, N, static_cast<int>(c.hidden), halves, unscale,
+                                                  halves_by_line(logits_w, N), s);
     // Large logits (8 MiB and up, unsplit Q8_0) are computed in bands of row
     // tiles, each copied to the host while the next is computed.
     LogitsBands b;

@@ -75,7 +75,10 @@ void launch_batch_product(const Weight& w, const float* x, const _Float16* halve
 // bands
 void launch_batch_product_tiles(const Weight& w, int tile0, int tile1, const _Float16* halves, const float* unscale,
                                 int n, float* out, hipStream_t s);
-void launch_split_halves(const float* x, int n, int cols, _Float16* halves, float* unscale, hipStream_t s);
+// the order of the halves that the product of n vectors reads
+bool halves_by_line(const Weight& w, int n);
+void launch_split_halves(const float* x, int n, int cols, _Float16* halves, float* unscale, bool by_line,
+                         hipStream_t s);
 void launch_split_sum(const float* p, int splits, int n, int rows, float* out, hipStream_t s);
 // the split sums of the fused QKV product into q, k (rotated by row j's
 // (cos, sin) at cs + j*dim) and v
@@ -84,10 +87,10 @@ void launch_qkv_epilogue(const float* p, int splits, int n, int qheads, int khea
 // x += the split sums (p may be null), then RMSNorm into norm and, when
 // halves is given, into the next product's halves
 void launch_resid_norm(const float* p, int splits, float* x, const float* w, int n, int h, float eps, float* norm,
-                       _Float16* halves, float* unscale, hipStream_t s);
+                       _Float16* halves, float* unscale, bool by_line, hipStream_t s);
 // SwiGLU of the fused gate|up sums into out and, when given, halves
 void launch_swiglu_epilogue(const float* p, int splits, int n, int inter, float* out, _Float16* halves,
-                            float* unscale, hipStream_t s, bool interleaved);
+                            float* unscale, bool by_line, hipStream_t s, bool interleaved);
 // out[j] = row idx[j] (or `row` when idx is null) of a Q8_0 table, dequantised
 void launch_gather_embedding_q8(const Weight& w, const uint32_t* idx, uint32_t row, int n, float* out,
                                 hipStream_t s);

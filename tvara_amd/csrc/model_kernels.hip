@@ -556,9 +556,17 @@ __global__ __launch_bounds__(W * 64) void matvec_q8_kernel(const Q8MatvecArgs a)
 // [2^13, 2^14), exact) and split as x = hi + lo with hi = fp16(x) and
 // lo = fp16(x - hi), which keeps 22 of its 24 bits.  One 16x16x32 MFMA then
 // covers exactly one Q8_0 group: C = A*Bhi + A*Blo in f32, and the
-// accumulator takes d * C.  Element k of vector j sits where lane
-// (j%16) + 16((k%32)/8) of vector tile j/16 reads it as a B operand:
-// halves[((vt*groups + k/32)*2 + part)*64 + lane][k%8], part 0 = hi, 1 = lo.
+// accumulator takes d * C.  A lane l of a product reads 16 bytes, columns
+// 8(l/16) .. +7 of vector l%16 of a tile.  Two orders:
+//  by lane, where the chunked kernel reads them straight into registers:
+//    halves[((vt*groups + k/32)*2 + part)*64 + lane][k%8], part 0 = hi, 1 = lo
+//    (in the other order its reads touch sixteen lines an instruction: 10.6
+//    against 15.9 us for 64 vectors of the 2,048-column products);
+//  by line, where the tiled GEMM stages them: a vector's halves of a group are
+//    128 contiguous bytes, halves[((vt*groups + k/32)*16 + j%16)*2 + part][k%32],
+//    so that an epilogue, a workgroup per vector, writes whole lines (by lane
+//    every line is written in pieces by eight workgroups: the SwiGLU of 2,048
+//    vectors of 8,192 takes 87 us against 49, the norms 24 against 16).
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef float float4v __attribute__((ext_vector_type(4)));
@@ -566,17 +574,17 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // Elements k0 .. k0 + 7 of vector j (k0 % 8 == 0, already scaled): one
 // 16-byte store each for the hi and the lo halves
-__device__ __forceinline__ void put_halves8(_Float16* halves, int groups, int j, int k0, const float (&v)[8]) {
+__device__ __forceinline__ void put_halves8(_Float16* halves, int groups, bool by_line, int j, int k0, const float (&v)[8]) {
     half8 hi, lo;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
         hi[i] = static_cast<_Float16>(v[i]);
         lo[i] = static_cast<_Float16>(v[i] - static_cast<float>(hi[i]));
     }
-    const int lane = (j % 16) + 16 * ((k0 % 32) / 8);
-    const size_t at = ((static_cast<size_t>(j / 16) * groups + k0 / 32) * 2 * 64 + lane) * 8;
+    const size_t block = (static_cast<size_t>(j / 16) * groups + k0 / 32) * 1024;  // of a vector tile and group
+    const size_t at = block + (by_line ? (j % 16) * 64 + k0 % 32 : ((j % 16) + 16 * ((k0 % 32) / 8)) * 8);
     *reinterpret_cast<half8*>(halves + at) = hi;
-    *reinterpret_cast<half8*>(halves + at + 64 * 8) = lo;
+    *reinterpret_cast<half8*>(halves + at + (by_line ? 32 : 512)) = lo;
 }
 
 __device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
@@ -621,7 +629,7 @@ inline int epi_threads(int h) { return std::min(1024, std::max(64, ((h / 8 + 63)
 
 // halves of vector j = blockIdx.x (a row of cols floats)
 __global__ __launch_bounds__(1024) void split_halves_kernel(const float* x, int cols, int groups, _Float16* halves,
-                                                             float* unscale) {
+                                                             float* unscale, bool by_line) {
     __shared__ float part[16];
     const int j = blockIdx.x, T = blockDim.x;
     const float* xr = x + static_cast<size_t>(j) * cols;
@@ -645,7 +653,7 @@ __global__ __launch_bounds__(1024) void split_halves_kernel(const float* x, int 
         if (e0 < cols) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[c][i] *= up;
-            put_halves8(halves, groups, j, e0, v[c]);
+            put_halves8(halves, groups, by_line, j, e0, v[c]);
         }
     }
 }
@@ -857,10 +865,10 @@ __global__ __launch_bounds__(256) void batch_q8_kernel(const Q8BatchArgs a) {
 // split, a wave VT by four of them, so that the operands a wave reads from LDS
 // per group, (2*VT + 4) KiB, feed 8*VT MFMAs.  K advances a group pair a step,
 // two steps ahead of the products: the activation halves go from memory
-// straight into one of three LDS buffers (16 bytes a lane, in the operand
-// order they are stored in), the int8 weights into one of two register sets
-// and from there, converted once for the workgroup, into one of two LDS
-// buffers; the scales a lane needs stay in registers.  A step has one barrier.
+// straight into one of three LDS buffers (16 bytes a lane, in operand order),
+// the int8 weights into one of two register sets and from there, converted
+// once for the workgroup, into one of two LDS buffers; the scales a lane needs
+// stay in registers.  A step has one barrier.
 // With VT = 4 the buffers take all 160 KB of LDS: one workgroup a CU, two
 // waves a SIMD.
 // Workgroups are numbered so that each XCD takes a contiguous run of tiles
@@ -910,7 +918,7 @@ __global__ __launch_bounds__(512, 2) void batch_q8_pipe_kernel(const Q8BatchArgs
                                            static_cast<uint32_t>(tiles_here * a.pairs) * 64u);
     const __amdgpu_buffer_rsrc_t xv =
         view(a.halves, static_cast<uint32_t>(a.n_total_tiles) * static_cast<uint32_t>(a.groups) * 2048u);
-    const uint32_t xoff = static_cast<uint32_t>(lane) * 16u;
+    const uint32_t xoff = static_cast<uint32_t>((lane & 15) * 128 + (lane >> 4) * 16);
     const uint32_t qoff = static_cast<uint32_t>((wave * a.pairs * 64 + lane) * 16);  // row tiles wave, wave + 8
     const uint32_t doff = static_cast<uint32_t>((rh * 4 * a.pairs * 16 + (lane & 15)) * 4);
 
@@ -931,7 +939,7 @@ __global__ __launch_bounds__(512, 2) void batch_q8_pipe_kernel(const Q8BatchArgs
             const int t = (wave * XL + i) / 4, part = (wave * XL + i) % 4;
             const int vt = min(vb * BV + t, a.n_total_tiles - 1);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(xv, (__attribute__((address_space(3))) void*)&x[t][part][0], 16, xoff,
-                                                     (vt * a.groups + 2 * (pbeg + p)) * 2048 + part * 1024, 0, 0);
+                                                     (vt * a.groups + 2 * (pbeg + p) + part / 2) * 2048 + part % 2 * 64, 0, 0);
         }
     };
     auto stage = [&](const uint4 (&raw)[2], half8 (&ws)[2][BR][64]) {
@@ -1110,7 +1118,7 @@ __global__ void qkv_epilogue_kernel(const float* p, int splits, int n, int qhead
 // its chunks in registers between the passes.
 __global__ __launch_bounds__(1024) void resid_norm_kernel(const float* p, int splits, float* x, const float* w, int n,
                                                           int h, float eps, float* norm, _Float16* halves, int groups,
-                                                          float* unscale) {
+                                                          float* unscale, bool by_line) {
     __shared__ double part[16];
     __shared__ float mpart[16];
     const int j = blockIdx.x, T = blockDim.x;
@@ -1164,7 +1172,7 @@ __global__ __launch_bounds__(1024) void resid_norm_kernel(const float* p, int sp
         if (e0 < h) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) y[c][i] *= up;
-            put_halves8(halves, groups, j, e0, y[c]);
+            put_halves8(halves, groups, by_line, j, e0, y[c]);
         }
     }
 }
@@ -1174,7 +1182,7 @@ __global__ __launch_bounds__(1024) void resid_norm_kernel(const float* p, int sp
 // product's halves
 __global__ __launch_bounds__(1024) void swiglu_epilogue_kernel(const float* p, int splits, int n, int inter, float* out,
                                                                _Float16* halves, int groups, float* unscale,
-                                                               int interleaved) {
+                                                               int interleaved, bool by_line) {
     __shared__ float mpart[16];
     const int j = blockIdx.x, T = blockDim.x;
     const size_t stride = static_cast<size_t>(n) * 2 * inter, base = static_cast<size_t>(j) * 2 * inter;
@@ -1219,7 +1227,7 @@ __global__ __launch_bounds__(1024) void swiglu_epilogue_kernel(const float* p, i
         if (e0 < inter) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) val[c][i] *= up;
-            put_halves8(halves, groups, j, e0, val[c]);
+            put_halves8(halves, groups, by_line, j, e0, val[c]);
         }
     }
 }
@@ -1480,6 +1488,8 @@ void launch_pipe(const Weight& w, const PipePlan& p, int tile0, int tile1, const
 }
 }  // namespace
 
+bool halves_by_line(const Weight& w, int n) { return pipe_for(w, n); }
+
 int batch_splits(const Weight& w, int n) {
     if (!w.q8) return f32_plan(w.rows, w.cols).splits;
     return pipe_for(w, n) ? pipe_plan(w, n, w.tiles()).splits : q8_plan(w).splits;
@@ -1577,10 +1587,11 @@ void launch_batch_product_tiles(const Weight& w, int tile0, int tile1, const _Fl
     TVARA_HIP(hipGetLastError());
 }
 
-void launch_split_halves(const float* x, int n, int cols, _Float16* halves, float* unscale, hipStream_t s) {
+void launch_split_halves(const float* x, int n, int cols, _Float16* halves, float* unscale, bool by_line,
+                         hipStream_t s) {
     if (cols % 32 || cols > 1024 * 8 * kEpiChunks) throw std::invalid_argument("batched decode width above 16384");
     launch("model_split_halves", split_halves_kernel, dim3(n), dim3(epi_threads(cols)), 0, s, x, cols, cols / 32, halves,
-           unscale);
+           unscale, by_line);
     TVARA_HIP(hipGetLastError());
 }
 
@@ -1593,18 +1604,18 @@ void launch_qkv_epilogue(const float* p, int splits, int n, int qheads, int khea
 }
 
 void launch_resid_norm(const float* p, int splits, float* x, const float* w, int n, int h, float eps, float* norm,
-                       _Float16* halves, float* unscale, hipStream_t s) {
+                       _Float16* halves, float* unscale, bool by_line, hipStream_t s) {
     if (h % 32 || h > 1024 * 8 * kEpiChunks) throw std::invalid_argument("batched decode width above 16384");
     launch("model_resid_norm", resid_norm_kernel, dim3(n), dim3(epi_threads(h)), 0, s, p, splits, x, w, n, h, eps, norm,
-           halves, h / 32, unscale);
+           halves, h / 32, unscale, by_line);
     TVARA_HIP(hipGetLastError());
 }
 
 void launch_swiglu_epilogue(const float* p, int splits, int n, int inter, float* out, _Float16* halves,
-                            float* unscale, hipStream_t s, bool interleaved) {
+                            float* unscale, bool by_line, hipStream_t s, bool interleaved) {
     if (inter % 32 || inter > 1024 * 8 * kEpiChunks) throw std::invalid_argument("batched decode width above 16384");
     launch("model_swiglu_epilogue", swiglu_epilogue_kernel, dim3(n), dim3(epi_threads(inter)), 0, s, p, splits, n, inter,
-           out, halves, inter / 32, unscale, interleaved ? 1 : 0);
+           out, halves, inter / 32, unscale, interleaved ? 1 : 0, by_line);
     TVARA_HIP(hipGetLastError());
 }
 
