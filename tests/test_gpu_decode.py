@@ -749,3 +749,49 @@ def test_wave_split_chunks_against_reference(device, oracle, dim, kv_heads, grou
     say("wave-split row", dim, kv_heads, group, length)
     got, want = _single(device, oracle, kv_heads * group, kv_heads, dim, 16, length, seed=length + dim, tail=True)
     assert refmath.close(got, want, TOL), refmath.max_rel(got, want)
+
+
+def test_closed_plans_buffers_serve_new_plans(device, oracle):
+    # plans made and closed in a loop, unchecked and unsynchronised, as a
+    # serving loop makes them: a launch in flight keeps its tables, partials and
+    # flag (its output is the one that a plan held open gives), a non-finite
+    # score of a closed plan fails no other, a plan on another stream and one
+    # that outlives its cache close cleanly
+    from tvara_amd import hip
+
+    heads, kv_heads, dim, tpb = 32, 8, 64, 16
+    w = kv_heads * dim
+    dev = device.PagedCache(1, kv_heads, dim, tpb, 400)
+    lengths = [700, 33, 512, 1, 1040, 300]
+    seqs = []
+    for i, n in enumerate(lengths):
+        seqs.append(dev.create_sequence())
+        dev.append_many(seqs[i], synth.normal(60 + i, "k", n * w).reshape(n, w),
+                        synth.normal(60 + i, "v", n * w).reshape(n, w))
+    subsets = [seqs, seqs[:1], seqs[2:], seqs[1:4], seqs[4:]]
+    want, q, outs = [], [], []
+    for i, part in enumerate(subsets):
+        q.append(synth.normal(70 + i, "q", len(part) * heads * dim).reshape(len(part), heads * dim))
+        want.append(attention.decode_batch(dev, q[i], part, 0, heads, 4096))
+    dq = [hip.DeviceArray.from_numpy(x) for x in q]
+    poison = hip.DeviceArray.from_numpy(np.full_like(q[0], np.nan))
+    sink = hip.DeviceArray(q[0].shape)
+    for r in range(4 * len(subsets)):
+        i = r % len(subsets)
+        outs.append((i, hip.DeviceArray(q[i].shape)))
+        attention.DecodePlan(dev, subsets[i], heads, 4096).launch(0, dq[i].ptr, outs[-1][1].ptr)
+        attention.DecodePlan(dev, seqs, heads, 4096).launch(0, poison.ptr, sink.ptr)  # closed unchecked
+    for i, out in outs:
+        assert np.array_equal(out.numpy(), want[i]), i
+    stream = hip.Stream(non_blocking=True)
+    for r in range(6):
+        plan = attention.DecodePlan(dev, seqs, heads, 4096)
+        plan.launch(0, dq[0].ptr, sink.ptr, stream=stream.h if r % 2 else None)
+        plan.check()
+        assert np.array_equal(sink.numpy(), want[0]), r
+        if r % 3:
+            plan.close()
+    held = attention.DecodePlan(dev, seqs, heads, 4096)
+    held.launch(0, dq[0].ptr, sink.ptr)
+    dev.close()
+    held.close()

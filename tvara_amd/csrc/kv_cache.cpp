@@ -118,6 +118,7 @@ DeviceCache::DeviceCache(const Geometry& g, int format) : meta_(g), format_(form
 }
 
 DeviceCache::~DeviceCache() {
+    plans_->close();
     (void)hipStreamSynchronize(stream_);
     for (hipEvent_t e : ordered_)
         if (e) (void)hipEventDestroy(e);
@@ -555,13 +556,69 @@ void AttnPlan::xcd_balance(int xcds) {
     order.n = n;
 }
 
+AttnPlan::~AttnPlan() {
+    if (buf && home && null_stream) home->give(std::move(buf));
+}
+
 void AttnPlan::place() {
     size_t copied = 0;
     const size_t total = region_bytes(&copied);
-    char* device = static_cast<char*>(region.ensure(total));
-    char* host = static_cast<char*>(staging.acquire(copied));
-    place_in(device, region.bytes, cache->stream(), host);
-    staging.release(cache->stream());
+    hipStream_t s = cache->stream();
+    null_stream &= s == nullptr;
+    if (!buf) {
+        home = cache->plan_pool();
+        buf = s ? std::make_unique<PlanPool::Set>() : home->take(total);
+    }
+    char* device = static_cast<char*>(buf->region.ensure(total));
+    char* host = static_cast<char*>(buf->staging.acquire(copied));
+    place_in(device, buf->region.bytes, s, host);
+    buf->staging.release(s);
+}
+
+PlanPool::Set::~Set() {
+    if (idle) (void)hipEventDestroy(idle);
+}
+
+std::unique_ptr<PlanPool::Set> PlanPool::take(size_t bytes) {
+    std::unique_ptr<Set> out;
+    {
+        std::lock_guard<std::mutex> hold(lock_);
+        size_t best = sets_.size();
+        for (size_t i = 0; i < sets_.size(); ++i)
+            if (sets_[i]->region.bytes >= bytes && (best == sets_.size() || sets_[i]->region.bytes < sets_[best]->region.bytes) &&
+                hipEventQuery(sets_[i]->idle) == hipSuccess)
+                best = i;
+        (void)hipGetLastError();  // (not ready is no error)
+        if (best < sets_.size()) {
+            out = std::move(sets_[best]);
+            sets_.erase(sets_.begin() + static_cast<std::ptrdiff_t>(best));
+        }
+    }
+    return out ? std::move(out) : std::make_unique<Set>();
+}
+
+void PlanPool::give(std::unique_ptr<Set> s) {
+    // (an event of another device than the current one fails to record)
+    if (s->region.bytes <= kSetBytes &&
+        (s->idle || hipEventCreateWithFlags(&s->idle, hipEventDisableTiming) == hipSuccess) &&
+        hipEventRecord(s->idle, nullptr) == hipSuccess) {
+        std::lock_guard<std::mutex> hold(lock_);
+        if (!closed_) {
+            sets_.push_back(std::move(s));
+            if (sets_.size() > kSets) {
+                s = std::move(sets_.front());  // the oldest goes
+                sets_.erase(sets_.begin());
+            }
+        }
+    }
+    // what is left in s is freed here, outside the lock (hipFree waits for its work)
+}
+
+void PlanPool::close() {
+    std::vector<std::unique_ptr<Set>> rest;
+    std::lock_guard<std::mutex> hold(lock_);
+    closed_ = true;
+    rest.swap(sets_);
 }
 
 namespace {
@@ -657,27 +714,28 @@ void AttnPlan::launch(int layer, const float* q, const float* tail_k, const floa
     a.ws_chunks = ws_chunks;
     a.row_major = row_major ? 1 : 0;
     a.qscale = static_cast<float>(1.4426950408889634 / std::sqrt(static_cast<double>(cache->geometry().head_dim)));
-    a.err = pinned_err ? static_cast<int*>(flag.ptr) : dev.err;
+    a.err = pinned_err ? static_cast<int*>(buf->flag.ptr) : dev.err;
     launch_decode(a, items, rows, need_merge, inline_ok ? &inline_rows : nullptr, order.n ? &order : nullptr, s,
                   ws_items.n ? &ws_items : nullptr);
     cache->leave(s);
     last_stream = s;
+    null_stream &= s == nullptr;
 }
 
 void AttnPlan::use_pinned_error() {
     if (pinned_err) return;
-    *static_cast<volatile int*>(flag.acquire(sizeof(int))) = 0;
+    *static_cast<volatile int*>(buf->flag.acquire(sizeof(int))) = 0;
     pinned_err = true;
 }
 
 void AttnPlan::queue_check() {
     if (pinned_err) return;  // the kernels write the pinned flag themselves
-    auto* f = static_cast<int*>(flag.acquire(sizeof(int)));
+    auto* f = static_cast<int*>(buf->flag.acquire(sizeof(int)));
     TVARA_HIP(hipMemcpyAsync(f, dev.err, sizeof(int), hipMemcpyDeviceToHost, last_stream));
 }
 
 void AttnPlan::finish_check() {
-    auto* f = static_cast<volatile int*>(flag.ptr);
+    auto* f = static_cast<volatile int*>(buf->flag.ptr);
     if (*f) {
         if (pinned_err) {
             *f = 0;
