@@ -672,3 +672,28 @@ def test_f32_tiles_non_finite(device, dim):
     kb[at, 3] = np.inf
     with pytest.raises(ValueError, match="invalid online attention input"):
         run(kb, v)
+
+
+@pytest.mark.parametrize("precision", ["bf16", "f32x3"])
+@pytest.mark.parametrize("fmt", ["f32", "q8_0"])
+@pytest.mark.parametrize("dim", [64, 128])
+@pytest.mark.parametrize("group,tpb", [(1, 16), (3, 64), (4, 16), (8, 1024), (12, 16)])
+def test_tile_key_splits(device, oracle, group, tpb, dim, fmt, precision):
+    # few workgroups, so their key tiles run as splits: a chunk whose last split
+    # takes the rest of the keys, chunks of one split beside it (written without
+    # a merge), and a chunk whose rows start mid-tile; every row against the
+    # oracle, with the bars of the short rows (above)
+    heads, kv_heads = 2 * group, 2
+    specs = [(2615, 2500, 100), (300, 0, 300), (70, 67, 3), (1, 0, 1), (1000, 865, 135)]
+    say("prefill splits", precision, "group", group, "tpb", tpb, "dim", dim, fmt)
+    dev, ref, ds, rs, qs = build(device, oracle, heads, kv_heads, dim, specs, seed=120 + group, tpb=tpb, q8=fmt == "q8_0")
+    starts = [s for _, s, _ in specs]
+    counts = [r for _, _, r in specs]
+    got = attention.prefill_batch(dev, np.concatenate(qs), ds, starts, counts, 0, heads, 4096, precision=precision)
+    want = np.concatenate([ref.fused_prompt_attention(q, s, 0, st, c, heads, 4096).reshape(c, -1)
+                           for q, s, st, c in zip(qs, rs, starts, counts)])
+    if precision == "bf16":
+        ok, err = bf16_ok(got, want, SHORT_ROWS)
+        assert ok, err
+    else:
+        assert refmath.close(got, want, TOL_F32), refmath.max_rel(got, want)

@@ -145,7 +145,8 @@ struct PrefillArgs {
     const int32_t* tables;
     // two entries a workgroup, by blockIdx.x (PrefillPlan::build): the
     // sequence (x: table offset, y: start, z: rows, w: first query row), then
-    // x: KV head, y: first chunk position, z: first key tile (f32 tiles)
+    // x: KV head | split << 16, y: first chunk position, z, w: first key tile and
+    // one past the last
     const int4* work;
     int workgroups;  // a multiple of eight; the lists' padding has no rows
     const float* q;    // [sum rows][heads][head_dim]
@@ -155,10 +156,11 @@ struct PrefillArgs {
     // as DecodeArgs::kv_share: lay.kv_heads and group describe kv_share
     // virtual KV heads per KV head (GQA groups above eight)
     int kv_share;
-    // f32 tiles: the key tiles are cut into `splits` runs of split_tiles, whose
-    // partial outputs, [split][row][heads][head_dim], and (maximum in log2
-    // units, normaliser) pairs, [split][row][heads][2], a second kernel merges
+    // the key tiles are cut into up to `splits` runs, whose partial outputs, [split][row][heads][head_dim], and
+    // (maximum in log2 units, normaliser) pairs, [split][row][heads][2], a
+    // second kernel merges; the bf16 tiles' rows have row_splits[row] of them
     int splits, split_tiles, total_rows;
+    const int* row_splits;
     float* part_acc;
     float* part_ml;
 };
@@ -208,6 +210,8 @@ bool prefill_bf16_supported(const BlockLayout& lay, int group);
 bool prefill_x3_supported(const BlockLayout& lay, int group);
 void launch_prefill_bf16(const PrefillArgs& a, hipStream_t s, bool x3 = false);
 int prefill_bf16_positions(int group);  // chunk positions of a workgroup
+// the splits of a row combined into a.out (prefill_f32.hip)
+void launch_prefill_merge(const PrefillArgs& a, hipStream_t s);
 // prefill_f32.hip: the same layouts in f32
 void launch_prefill_f32(const PrefillArgs& a, hipStream_t s);
 int prefill_f32_positions(const BlockLayout& lay, int group);

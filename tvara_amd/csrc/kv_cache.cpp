@@ -774,6 +774,34 @@ void AttnPlan::check_after(hipEvent_t after) {
     finish_check();
 }
 
+// A chunk with fewer workgroups than CUs (a CU runs one at a time) leaves the
+// rest idle, down to eight workgroups that walk all the keys: its key tiles are
+// cut into about one run a CU, of at least four tiles.  MI355X, unsplit against
+// split: 64 tokens after 8,000 at 32 x 8 heads of 64 151.8 -> 23.7 us (bf16)
+// and 314 -> 30.3 (three products), 512 after 2,000 56.3 -> 32.5, 256 after
+// 2,000 at heads of 128, three products, 168.5 -> 51.2, 900 after 1,000 over
+// Q8_0 77.2 -> 59.9.  From 256 workgroups on a split only adds rounds (256
+// of 200-260 tiles: 547 us against 770 in 512 units and 602 in 1,024).
+void PrefillPlan::bf16_splits(const std::vector<int4>& seqs, int kv_heads, int positions) {
+    constexpr int64_t kUnits = 256;
+    int64_t wgs = 0, total = 0;
+    int longest = 0;
+    for (const int4& q : seqs) {
+        const int all = (q.y + q.z + 63) / 64, n = (q.z + positions - 1) / positions;
+        wgs += n;
+        total += static_cast<int64_t>(n) * all;
+        longest = std::max(longest, all);
+    }
+    wgs *= kv_heads;
+    total *= kv_heads;
+    splits = 1;
+    split_tiles = longest;
+    if (wgs >= kUnits) return;
+    split_tiles = static_cast<int>(
+        std::min<int64_t>(std::max<int64_t>({4, (total + kUnits - 1) / kUnits, (longest + 1023) / 1024}), longest));
+    splits = (longest + split_tiles - 1) / split_tiles;
+}
+
 // The tile kernels' workgroups.  Ids go to the eight XCDs round-robin and,
 // within an XCD, to its shader engines in turn, each id waiting for its
 // engine: ids in order of (chunk tile, sequence), many of them empty for a
@@ -783,11 +811,11 @@ void AttnPlan::check_after(hipEvent_t after) {
 // XCD's L2, and each XCD's run is ordered from the most keys to the fewest
 // (MI355X, four chunks of 200-900 tokens after 500-3,000 at head_dim 128 on
 // the three-product tiles: 439 -> 261 us; even batches unchanged).
-std::vector<int4> PrefillPlan::work_list(const std::vector<int4>& seqs, int kv_heads, int positions) const {
+std::vector<int4> PrefillPlan::work_list(const std::vector<int4>& seqs, int kv_heads, int positions,
+                                         std::vector<int>& row_runs) const {
     constexpr int kXcds = 8, kCus = 32, kTileKeys = 64;
     struct Item {
-        int seq, head, q0, tile0;
-        int64_t tiles;
+        int seq, head, q0, split, tile0, end;
     };
     std::vector<Item> items, empty;
     int64_t total = 0;
@@ -796,14 +824,23 @@ std::vector<int4> PrefillPlan::work_list(const std::vector<int4>& seqs, int kv_h
         for (int h = 0; h < kv_heads; ++h)
             for (int q0 = (rows - 1) / positions * positions; q0 >= 0; q0 -= positions) {
                 const int all = (start + std::min(q0 + positions, rows) + kTileKeys - 1) / kTileKeys;
-                for (int s = 0; s < splits; ++s) {
-                    const int t0 = s * split_tiles;
-                    const int64_t t = splits == 1 ? all : std::max(0, std::min(split_tiles, all - t0));
-                    (t ? items : empty).push_back({i, h, q0, t0, t});
-                    total += t;
+                if (precision == 0) {
+                    for (int s = 0; s < splits; ++s) {
+                        const int t0 = s * split_tiles, t1 = splits == 1 ? all : std::min(all, t0 + split_tiles);
+                        (t1 > t0 ? items : empty).push_back({i, h, q0, s, t0, std::max(t0, t1)});
+                    }
+                } else {
+                    // the last run starts where every row still sees a key
+                    const int most = (start + q0) / kTileKeys / split_tiles + 1;
+                    const int runs = std::min({splits, (all + split_tiles - 1) / split_tiles, most});
+                    for (int s = 0; s < runs; ++s)
+                        items.push_back({i, h, q0, s, s * split_tiles, s + 1 == runs ? all : (s + 1) * split_tiles});
+                    if (splits > 1)
+                        std::fill_n(row_runs.begin() + seqs[i].w + q0, std::min(positions, rows - q0), runs);
                 }
             }
     }
+    for (const Item& it : items) total += it.end - it.tile0;
     // up to four rounds of the CUs, no XCD takes more workgroups than its CUs
     // need rounds for: one more would add a whole round (256 workgroups of
     // 200-250 tiles, 33 of them on one XCD: 1,003 against 548 us)
@@ -815,10 +852,10 @@ std::vector<int4> PrefillPlan::work_list(const std::vector<int4>& seqs, int kv_h
         const bool full = static_cast<int64_t>(run[x].size()) == cap, share = before * kXcds >= total * (x + 1);
         if (x + 1 < kXcds && (full || (share && count - i <= cap * (kXcds - 1 - x)))) ++x;
         run[x].push_back(items[i]);
-        before += items[i].tiles;
+        before += items[i].end - items[i].tile0;
     }
     for (auto& r : run)
-        std::stable_sort(r.begin(), r.end(), [](const Item& a, const Item& b) { return a.tiles > b.tiles; });
+        std::stable_sort(r.begin(), r.end(), [](const Item& a, const Item& b) { return a.end - a.tile0 > b.end - b.tile0; });
     // splits without keys write that they have none
     for (size_t i = 0; i < empty.size(); ++i) run[i % kXcds].push_back(empty[i]);
     size_t longest = 0;
@@ -830,7 +867,7 @@ std::vector<int4> PrefillPlan::work_list(const std::vector<int4>& seqs, int kv_h
         for (size_t k = 0; k < run[r].size(); ++k) {
             const Item& it = run[r][k];
             list[2 * (k * kXcds + r)] = seqs[it.seq];
-            list[2 * (k * kXcds + r) + 1] = make_int4(it.head, it.q0, it.tile0, 0);
+            list[2 * (k * kXcds + r) + 1] = make_int4(it.head | it.split << 16, it.q0, it.tile0, it.end);
         }
     return list;
 }
@@ -903,10 +940,14 @@ void PrefillPlan::build(DeviceCache* c, const uint64_t* sequences, size_t n, siz
     }
     if (tab.size() > static_cast<size_t>(std::numeric_limits<int32_t>::max()))
         throw std::invalid_argument("attention batch too large");
-    const std::vector<int4> list = work_list(sq, static_cast<int>(g.kv_heads) * kv_share,
-                                             prec == 0 ? prefill_f32_positions(c->layout(), group / kv_share)
-                                                       : prefill_bf16_positions(group / kv_share));
+    const int qt = prec == 0 ? prefill_f32_positions(c->layout(), group / kv_share) : prefill_bf16_positions(group / kv_share);
+    if (prec != 0) bf16_splits(sq, static_cast<int>(g.kv_heads) * kv_share, qt);
+    std::vector<int> row_runs(prec != 0 && splits > 1 ? total_rows : 0);
+    std::vector<int4> list = work_list(sq, static_cast<int>(g.kv_heads) * kv_share, qt, row_runs);
     workgroups = static_cast<int>(list.size() / 2);
+    runs_at = list.size();
+    list.resize(runs_at + (row_runs.size() + 3) / 4);
+    if (!row_runs.empty()) std::memcpy(list.data() + runs_at, row_runs.data(), row_runs.size() * sizeof(int));
     void* pt = tables.ensure(std::max<size_t>(tab.size() * sizeof(int32_t), 16));
     void* pw = work.ensure(list.size() * sizeof(int4));
     void* pe = err.ensure(sizeof(int));
@@ -942,17 +983,17 @@ void PrefillPlan::launch(int layer, const float* q, float* out, hipStream_t s) {
     a.out = out;
     a.qscale = static_cast<float>(1.4426950408889634 / std::sqrt(static_cast<double>(cache->geometry().head_dim)));
     a.err = pinned_err ? static_cast<int*>(flag.ptr) : static_cast<int*>(err.ptr);
-    if (precision == 0) {
-        a.splits = splits;
-        a.split_tiles = split_tiles;
-        a.total_rows = static_cast<int>(total_rows);
+    a.splits = splits;
+    a.total_rows = static_cast<int>(total_rows);
+    if (splits > 1) {
+        a.row_splits = precision == 0 ? nullptr : reinterpret_cast<const int*>(a.work + runs_at);
         a.part_acc = static_cast<float*>(part.ptr);
-        if (splits > 1)
-            a.part_ml = a.part_acc + static_cast<size_t>(splits) * total_rows * heads * cache->geometry().head_dim;
-        launch_prefill_f32(a, s);
-    } else {
-        launch_prefill_bf16(a, s, precision == 2);
+        a.part_ml = a.part_acc + static_cast<size_t>(splits) * total_rows * heads * cache->geometry().head_dim;
     }
+    if (precision == 0)
+        launch_prefill_f32(a, s);
+    else
+        launch_prefill_bf16(a, s, precision == 2);
     cache->leave(s);
     last_stream = s;
 }

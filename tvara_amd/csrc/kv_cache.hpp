@@ -268,7 +268,8 @@ struct PrefillPlan {
     bool on_rows = false;  // f32 through the decode kernels (rows_plan), not the tiles
     size_t total_rows = 0;
     AttnPlan rows_plan;
-    int splits = 1, split_tiles = 0;  // f32 tiles (prefill_f32_shape)
+    int splits = 1, split_tiles = 0;  // runs of key tiles per workgroup
+    size_t runs_at = 0;               // where the rows' counts of them start in `work`
     DeviceBuffer tables, work, err, part;
     // the tile kernels set the error flag in pinned host memory instead
     // (use_pinned_error: no copy back before a check)
@@ -281,7 +282,10 @@ struct PrefillPlan {
     void build(DeviceCache* c, const uint64_t* sequences, size_t count, size_t heads, size_t context,
                const size_t* start, const size_t* rows, int precision);
     // two entries a workgroup of the tile kernels (PrefillArgs::work)
-    std::vector<int4> work_list(const std::vector<int4>& seqs, int kv_heads, int positions) const;
+    std::vector<int4> work_list(const std::vector<int4>& seqs, int kv_heads, int positions,
+                                std::vector<int>& row_runs) const;
+    // splits and split_tiles of the bf16 and three-product tiles
+    void bf16_splits(const std::vector<int4>& seqs, int kv_heads, int positions);
     void use_pinned_error();
     void launch(int layer, const float* q, float* out, hipStream_t s);
     void check();

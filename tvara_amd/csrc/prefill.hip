@@ -100,12 +100,12 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_bf16_kernel(const Prefill
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int g = lane >> 4, r16 = lane & 15;
-    // the plan's work list (heaviest first within each XCD)
+    // the plan's work list (PrefillPlan::work_list: heaviest first within each XCD)
     const int4 sd = a.work[2 * blockIdx.x], wk = a.work[2 * blockIdx.x + 1];
-    const int start = sd.y, nrows = sd.z, kh = wk.x, q0 = wk.y;
+    const int start = sd.y, nrows = sd.z, kh = wk.x & 0xffff, q0 = wk.y;
     if (!nrows) return;  // the list's padding
     const int kmax = start + min(q0 + QT, nrows);  // keys this workgroup reads: [0, kmax)
-    const int ntiles = (kmax + kKeys - 1) / kKeys;
+    const int kt0 = wk.z, ntiles = wk.w;  // this workgroup's key tiles: every row sees the first key of kt0
     const int pw0 = q0 + wave * PW;
     const int wave_kmax = pw0 < nrows ? start + min(pw0 + PW, nrows) : 0;
     const int kvw = a.lay.kv_width;
@@ -452,15 +452,15 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_bf16_kernel(const Prefill
     };
     auto tile = [&](int t) { return min(t, ntiles - 1); };
     if constexpr (kStages == 2) {
-        tabload(0, bA);
-        gload(0, bA, kA, vA);
-        tabload(tile(1), bB);
-        gload(tile(1), bB, kB, vB);
-        tabload(tile(2), bA);
-        tabload(tile(3), bB);
-        lstore(0, 0, kA, vA);
+        tabload(kt0, bA);
+        gload(kt0, bA, kA, vA);
+        tabload(tile(kt0 + 1), bB);
+        gload(tile(kt0 + 1), bB, kB, vB);
+        tabload(tile(kt0 + 2), bA);
+        tabload(tile(kt0 + 3), bB);
+        lstore(kt0, 0, kA, vA);
         __syncthreads();
-        for (int kt = 0; kt < ntiles; kt += 2) {
+        for (int kt = kt0; kt < ntiles; kt += 2) {
             gload(tile(kt + 2), bA, kA, vA);
             tabload(tile(kt + 4), bA);
             compute(kt, 0);
@@ -475,16 +475,17 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_bf16_kernel(const Prefill
         }
     } else {
         // one register stage: tile t + 1 is requested before tile t's products
-        tabload(0, bA);
-        gload(0, bA, kA, vA);
-        tabload(tile(1), bA);
-        lstore(0, 0, kA, vA);
+        tabload(kt0, bA);
+        gload(kt0, bA, kA, vA);
+        tabload(tile(kt0 + 1), bA);
+        lstore(kt0, 0, kA, vA);
         __syncthreads();
-        for (int kt = 0; kt < ntiles; ++kt) {
+        for (int kt = kt0; kt < ntiles; ++kt) {
+            const int buf = (kt - kt0) & 1;
             gload(tile(kt + 1), bA, kA, vA);
             tabload(tile(kt + 2), bA);
-            compute(kt, kt & 1);
-            lstore(tile(kt + 1), (kt + 1) & 1, kA, vA);
+            compute(kt, buf);
+            lstore(tile(kt + 1), buf ^ 1, kA, vA);
             __syncthreads();
         }
     }
@@ -496,10 +497,19 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_bf16_kernel(const Prefill
         const float l = __shfl(acc[DT][nt][0], r16);
         const int r = 16 * nt + r16, pos = pw0 + r / G, head = kh * G + r % G;
         if (pos >= nrows || r >= PW * G) continue;
-        float* o = a.out + (static_cast<size_t>(sd.w + pos) * a.heads + head) * D + 4 * g;
+        size_t at = static_cast<size_t>(sd.w + pos) * a.heads + head;
+        float* o = a.out + at * D + 4 * g;
+        float div = l;
+        if (a.splits > 1 && a.row_splits[sd.w + pos] > 1) {  // a partial
+            at += static_cast<size_t>(wk.x >> 16) * a.total_rows * a.heads;
+            if (g == 0) *reinterpret_cast<float2*>(a.part_ml + 2 * at) = make_float2(m[nt], l);
+            o = a.part_acc + at * D + 4 * g;
+            bad |= !__builtin_isfinite(l);
+            div = 1.f;
+        }
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
-            const f32x4 v = acc[dt][nt] / l;
+            const f32x4 v = acc[dt][nt] / div;
             bad |= !__builtin_isfinite(v[0]) || !__builtin_isfinite(v[1]) || !__builtin_isfinite(v[2]) ||
                    !__builtin_isfinite(v[3]);
             *reinterpret_cast<float4*>(o + 16 * dt) = make_float4(v[0], v[1], v[2], v[3]);
@@ -871,12 +881,15 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_pipe_kernel(const Prefill
 // measured 158 against 225 us for four on the 8 x (2,048 + 512) chunk;
 // 128-key tiles 177 us).
 //
+// Key splits (PrefillPlan::bf16_splits) are the plain kernel's: a workgroup
+// then walks a run of the key tiles and leaves a partial.
+//
 // x3 (three products per product) always takes the plain kernel, over f32
 // or Q8_0 blocks (d * q dequantised when staged, then split).
 template <int D, int G, int TPB>
 void launch_gt(const PrefillArgs& b, bool x3, hipStream_t s) {
     const char* env = std::getenv("TVARA_PREFILL_PIPE");
-    const bool pipe = env ? std::atoi(env) != 0 : D == 64;
+    const bool pipe = b.splits == 1 && (env ? std::atoi(env) != 0 : D == 64);
     const bool q8 = b.lay.format == kQ8;
     constexpr int W = kWavesPerGroup;
     const dim3 grid(b.workgroups), block(64 * W);
@@ -939,6 +952,7 @@ void launch_prefill_bf16(const PrefillArgs& a, hipStream_t s, bool x3) {
         default: launch_g<8>(a, x3, s); break;
     }
     TVARA_HIP(hipGetLastError());
+    if (a.splits > 1) launch_prefill_merge(a, s);
 }
 
 }  // namespace tvara_amd

@@ -70,10 +70,10 @@ __global__ __launch_bounds__(64 * kRowsPerGroup / (16 * NT), 2) void prefill_f32
     const int G = a.group, PW = 16 * NT / G, QT = W * PW;  // positions per wave and workgroup
     // the plan's work list (heaviest first within each XCD)
     const int4 sd = a.work[2 * blockIdx.x], wk = a.work[2 * blockIdx.x + 1];
-    const int start = sd.y, nrows = sd.z, kh = wk.x, q0 = wk.y, kt0 = wk.z;
+    const int start = sd.y, nrows = sd.z, kh = wk.x & 0xffff, split = wk.x >> 16, q0 = wk.y, kt0 = wk.z;
     if (!nrows) return;  // the list's padding
     const int kmax = start + min(q0 + QT, nrows);
-    const int ntiles = min((kmax + kKeys - 1) / kKeys, kt0 + a.split_tiles);
+    const int ntiles = wk.w;
     const int pw0 = q0 + wave * PW;
     const int wave_kmax = pw0 < nrows ? start + min(pw0 + PW, nrows) : 0;
     const int kvw = a.lay.kv_width;
@@ -332,7 +332,7 @@ __global__ __launch_bounds__(64 * kRowsPerGroup / (16 * NT), 2) void prefill_f32
         float* o = a.out + at * D + 16 * g;
         float inv = total;
         if (a.splits > 1) {
-            at += static_cast<size_t>(kt0 / a.split_tiles) * a.total_rows * a.heads;
+            at += static_cast<size_t>(split) * a.total_rows * a.heads;
             if (g == 0) *reinterpret_cast<float2*>(a.part_ml + 2 * at) = make_float2(m[nt], total);
             if (m[nt] == -INFINITY) continue;  // no key of this split: not read either
             o = a.part_acc + at * D + 16 * g;
@@ -352,34 +352,36 @@ __global__ __launch_bounds__(64 * kRowsPerGroup / (16 * NT), 2) void prefill_f32
 // thread per four columns, all splits' loads of a round requested together.
 // Splits in which the row sees no key (maximum -inf) are left out.
 template <int D>
-__global__ __launch_bounds__(256) void prefill_f32_merge_kernel(const PrefillArgs a) {
+__global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillArgs a) {
     constexpr int U = 8;
     const size_t n = static_cast<size_t>(a.total_rows) * a.heads;
     const size_t t = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x, at = t / (D / 4);
     if (at >= n) return;
     const int c = 4 * static_cast<int>(t % (D / 4));
+    const int splits = a.row_splits ? a.row_splits[at / a.heads] : a.splits;
+    if (splits == 1 && a.row_splits) return;  // written by its one workgroup
     float M = -INFINITY, L = 0.f;
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < a.splits; s0 += U) {
+    for (int s0 = 0; s0 < splits; s0 += U) {
         float2 ml[U];
         f32x4 x[U];
 #pragma unroll
         for (int k = 0; k < U; ++k) {
-            const size_t p = static_cast<size_t>(min(s0 + k, a.splits - 1)) * n + at;
+            const size_t p = static_cast<size_t>(min(s0 + k, splits - 1)) * n + at;
             ml[k] = *reinterpret_cast<const float2*>(a.part_ml + 2 * p);
             x[k] = *reinterpret_cast<const f32x4*>(a.part_acc + p * D + c);
         }
         float mc = M;
 #pragma unroll
         for (int k = 0; k < U; ++k)
-            if (s0 + k < a.splits) mc = fmaxf(mc, ml[k].x);
+            if (s0 + k < splits) mc = fmaxf(mc, ml[k].x);
         if (mc == -INFINITY) continue;
         const float scale = fast_exp2(M - mc);  // 0 while M is -inf
         L *= scale;
         sum *= scale;
 #pragma unroll
         for (int k = 0; k < U; ++k) {
-            const bool some = s0 + k < a.splits && ml[k].x != -INFINITY;
+            const bool some = s0 + k < splits && ml[k].x != -INFINITY;
             const float w = some ? fast_exp2(ml[k].x - mc) : 0.f;
             L = fmaf(w, some ? ml[k].y : 0.f, L);
 #pragma unroll
@@ -409,12 +411,14 @@ void launch_prefill_f32(const PrefillArgs& a, hipStream_t s) {
         launch("paged_prefill_f32", q8 ? prefill_f32_kernel<64, 2, true> : prefill_f32_kernel<64, 2, false>, grid,
                dim3(256), 0, s, a);
     TVARA_HIP(hipGetLastError());
-    if (a.splits > 1) {
-        const size_t threads = static_cast<size_t>(a.total_rows) * a.heads * (a.lay.head_dim / 4);
-        launch("paged_prefill_f32_merge", wide ? prefill_f32_merge_kernel<128> : prefill_f32_merge_kernel<64>,
-               dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, s, a);
-        TVARA_HIP(hipGetLastError());
-    }
+    if (a.splits > 1) launch_prefill_merge(a, s);
+}
+
+void launch_prefill_merge(const PrefillArgs& a, hipStream_t s) {
+    const size_t threads = static_cast<size_t>(a.total_rows) * a.heads * (a.lay.head_dim / 4);
+    launch("paged_prefill_merge", a.lay.head_dim == 128 ? prefill_merge_kernel<128> : prefill_merge_kernel<64>,
+           dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, s, a);
+    TVARA_HIP(hipGetLastError());
 }
 
 int prefill_f32_positions(const BlockLayout& lay, int group) {
