@@ -581,7 +581,8 @@ typedef float float4v __attribute__((ext_vector_type(4)));
 
 // Elements k0 .. k0 + 7 of vector j (k0 % 8 == 0, already scaled): one
 // 16-byte store each for the hi and the lo halves
-__device__ __forceinline__ void put_halves8(_Float16* halves, int groups, bool by_line, int j, int k0, const float (&v)[8]) {
+template <bool kByLine>
+__device__ __forceinline__ void put_halves8(_Float16* halves, int groups, int j, int k0, const float (&v)[8]) {
     half8 hi, lo;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -589,9 +590,9 @@ __device__ __forceinline__ void put_halves8(_Float16* halves, int groups, bool b
         lo[i] = static_cast<_Float16>(v[i] - static_cast<float>(hi[i]));
     }
     const size_t block = (static_cast<size_t>(j / 16) * groups + k0 / 32) * 1024;  // of a vector tile and group
-    const size_t at = block + (by_line ? (j % 16) * 64 + k0 % 32 : ((j % 16) + 16 * ((k0 % 32) / 8)) * 8);
+    const size_t at = block + (kByLine ? (j % 16) * 64 + k0 % 32 : ((j % 16) + 16 * ((k0 % 32) / 8)) * 8);
     *reinterpret_cast<half8*>(halves + at) = hi;
-    *reinterpret_cast<half8*>(halves + at + (by_line ? 32 : 512)) = lo;
+    *reinterpret_cast<half8*>(halves + at + (kByLine ? 32 : 512)) = lo;
 }
 
 __device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
@@ -635,8 +636,9 @@ constexpr int kEpiChunks = 2;
 inline int epi_threads(int h) { return std::min(1024, std::max(64, ((h / 8 + 63) / 64) * 64)); }
 
 // halves of vector j = blockIdx.x (a row of cols floats)
+template <bool kByLine>
 __global__ __launch_bounds__(1024) void split_halves_kernel(const float* x, int cols, int groups, _Float16* halves,
-                                                             float* unscale, bool by_line) {
+                                                             float* unscale) {
     __shared__ float part[16];
     const int j = blockIdx.x, T = blockDim.x;
     const float* xr = x + static_cast<size_t>(j) * cols;
@@ -660,7 +662,7 @@ __global__ __launch_bounds__(1024) void split_halves_kernel(const float* x, int 
         if (e0 < cols) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) v[c][i] *= up;
-            put_halves8(halves, groups, by_line, j, e0, v[c]);
+            put_halves8<kByLine>(halves, groups, j, e0, v[c]);
         }
     }
 }
@@ -1123,9 +1125,10 @@ __global__ void qkv_epilogue_kernel(const float* p, int splits, int n, int qhead
 // scale rounded to float, (x * s) * w) into `norm` (when given) and, when
 // `halves` is given, into the next product's fp16 halves.  A thread keeps
 // its chunks in registers between the passes.
+template <bool kByLine>
 __global__ __launch_bounds__(1024) void resid_norm_kernel(const float* p, int splits, float* x, const float* w, int n,
                                                           int h, float eps, float* norm, _Float16* halves, int groups,
-                                                          float* unscale, bool by_line) {
+                                                          float* unscale) {
     __shared__ double part[16];
     __shared__ float mpart[16];
     const int j = blockIdx.x, T = blockDim.x;
@@ -1179,7 +1182,7 @@ __global__ __launch_bounds__(1024) void resid_norm_kernel(const float* p, int sp
         if (e0 < h) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) y[c][i] *= up;
-            put_halves8(halves, groups, by_line, j, e0, y[c]);
+            put_halves8<kByLine>(halves, groups, j, e0, y[c]);
         }
     }
 }
@@ -1187,9 +1190,10 @@ __global__ __launch_bounds__(1024) void resid_norm_kernel(const float* p, int sp
 // Vector j = blockIdx.x of the fused gate|up product: gate * (sigmoid(gate)
 // * up) (model.hpp:111-116) into `out` (when given) and, when given, the next
 // product's halves
+template <bool kByLine>
 __global__ __launch_bounds__(1024) void swiglu_epilogue_kernel(const float* p, int splits, int n, int inter, float* out,
                                                                _Float16* halves, int groups, float* unscale,
-                                                               int interleaved, bool by_line) {
+                                                               int interleaved) {
     __shared__ float mpart[16];
     const int j = blockIdx.x, T = blockDim.x;
     const size_t stride = static_cast<size_t>(n) * 2 * inter, base = static_cast<size_t>(j) * 2 * inter;
@@ -1234,7 +1238,7 @@ __global__ __launch_bounds__(1024) void swiglu_epilogue_kernel(const float* p, i
         if (e0 < inter) {
 #pragma unroll
             for (int i = 0; i < 8; ++i) val[c][i] *= up;
-            put_halves8(halves, groups, by_line, j, e0, val[c]);
+            put_halves8<kByLine>(halves, groups, j, e0, val[c]);
         }
     }
 }
@@ -1597,8 +1601,8 @@ void launch_batch_product_tiles(const Weight& w, int tile0, int tile1, const _Fl
 void launch_split_halves(const float* x, int n, int cols, _Float16* halves, float* unscale, bool by_line,
                          hipStream_t s) {
     if (cols % 32 || cols > 1024 * 8 * kEpiChunks) throw std::invalid_argument("batched decode width above 16384");
-    launch("model_split_halves", split_halves_kernel, dim3(n), dim3(epi_threads(cols)), 0, s, x, cols, cols / 32, halves,
-           unscale, by_line);
+    launch("model_split_halves", by_line ? split_halves_kernel<true> : split_halves_kernel<false>, dim3(n),
+           dim3(epi_threads(cols)), 0, s, x, cols, cols / 32, halves, unscale);
     TVARA_HIP(hipGetLastError());
 }
 
@@ -1613,16 +1617,16 @@ void launch_qkv_epilogue(const float* p, int splits, int n, int qheads, int khea
 void launch_resid_norm(const float* p, int splits, float* x, const float* w, int n, int h, float eps, float* norm,
                        _Float16* halves, float* unscale, bool by_line, hipStream_t s) {
     if (h % 32 || h > 1024 * 8 * kEpiChunks) throw std::invalid_argument("batched decode width above 16384");
-    launch("model_resid_norm", resid_norm_kernel, dim3(n), dim3(epi_threads(h)), 0, s, p, splits, x, w, n, h, eps, norm,
-           halves, h / 32, unscale, by_line);
+    launch("model_resid_norm", by_line ? resid_norm_kernel<true> : resid_norm_kernel<false>, dim3(n),
+           dim3(epi_threads(h)), 0, s, p, splits, x, w, n, h, eps, norm, halves, h / 32, unscale);
     TVARA_HIP(hipGetLastError());
 }
 
 void launch_swiglu_epilogue(const float* p, int splits, int n, int inter, float* out, _Float16* halves,
                             float* unscale, bool by_line, hipStream_t s, bool interleaved) {
     if (inter % 32 || inter > 1024 * 8 * kEpiChunks) throw std::invalid_argument("batched decode width above 16384");
-    launch("model_swiglu_epilogue", swiglu_epilogue_kernel, dim3(n), dim3(epi_threads(inter)), 0, s, p, splits, n, inter,
-           out, halves, inter / 32, unscale, interleaved ? 1 : 0, by_line);
+    launch("model_swiglu_epilogue", by_line ? swiglu_epilogue_kernel<true> : swiglu_epilogue_kernel<false>, dim3(n),
+           dim3(epi_threads(inter)), 0, s, p, splits, n, inter, out, halves, inter / 32, unscale, interleaved ? 1 : 0);
     TVARA_HIP(hipGetLastError());
 }
 
