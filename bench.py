@@ -34,8 +34,8 @@ host's CPU model, core count, compiler, flags, AVX2 use and a STREAM-style
 triad bandwidth.
 
 Other shapes, one line each with --workload: c4d128, c4q8 and c4f32 (the
-chunks at head_dim 128, over Q8_0 blocks, and in f32 through the decode
-kernels), c4x3 / c4x3d128 / c4q8x3 (the three-product tiles at f32
+chunks at head_dim 128, over Q8_0 blocks, and in f32 on the f32 matrix
+cores), c4x3 / c4x3d128 / c4q8x3 (the three-product tiles at f32
 accuracy), gqa8 / gqa8q8 (Llama-3-70B, eight query
 heads per KV head), gqa16 / gqa16q8 (Llama-3.1-405B, sixteen, run as two
 slices), tiny / tinyq8 (TinyLlama-1.1B), gemma2 (head_dim 256), phi3
@@ -442,9 +442,7 @@ FP32_PEAK_TFS = 157.3  # MI355X dense fp32 (matrix)
 def bench_prefill(args, w, precision="bf16"):
     """Chunked prefill: TFLOP/s over the algorithmic flops of the causal
     chunks.  bf16: the MFMA kernel.  f32 (the reference's arithmetic, within
-    1e-4): every chunk row runs as a decode row whose visible length stops at
-    its own position (attention.hpp:85-89), through the decode kernels and the
-    split merge; its dominant kernel is priced against the fp32 peak.  f32x3
+    1e-4): the tiles of the f32 matrix cores, priced against the fp32 peak.  f32x3
     (within the same 1e-4): the MFMA tiles with every operand split into two
     16-bit parts and three products per product, priced against a third of
     the 16-bit MFMA peak (the matrix rate left for the algorithmic flops)."""

@@ -256,10 +256,12 @@ struct AttnPlan {
 
 // Chunked-prefill plan: sequences[i] attends its prompt rows start[i] ..
 // start[i] + rows[i] - 1 causally (fused_prompt_attention,
-// attention.hpp:85-89).  precision 0 = f32 rows through the decode kernels,
-// 1 = the bf16 MFMA tile kernel, 2 = the tile kernel with three products
-// per product of split operands (f32 or Q8_0 blocks).  Block tables stay resident, so a plan built
-// once per chunk serves every layer.
+// attention.hpp:85-89).  precision 0 = f32: the f32 tile kernel, or rows
+// through the decode kernels where those are faster or the only ones
+// (prefill_f32_shape), 1 = the bf16 MFMA tile kernel, 2 = the tile kernel with
+// three products per product of split operands (f32 or Q8_0 blocks).  Block
+// tables and work lists stay resident, so a plan built once per chunk serves
+// every layer.
 struct PrefillPlan {
     DeviceCache* cache = nullptr;
     uint64_t epoch = 0;
