@@ -159,7 +159,7 @@ struct PrefillArgs {
     // the key tiles are cut into up to `splits` runs, whose partial outputs, [split][row][heads][head_dim], and
     // (maximum in log2 units, normaliser) pairs, [split][row][heads][2], a
     // second kernel merges; the bf16 tiles' rows have row_splits[row] of them
-    int splits, split_tiles, total_rows;
+    int splits, total_rows;
     const int* row_splits;
     float* part_acc;
     float* part_ml;
