@@ -234,6 +234,31 @@ def test_sequences_decode_matches_serial_reference(tmp_path, ref_capi, nseq, emb
     say("sequences_decode", nseq, "worst relative logit error", worst)
 
 
+@pytest.mark.parametrize("vocab", [32800, 34001])
+@pytest.mark.parametrize("nseq", [65, 130, 300])
+def test_many_sequences_logits_in_bands(tmp_path, nseq, vocab):
+    # above 64 sequences the logits are the tiled product's, computed in four
+    # bands of row tiles (2,050 and 2,126 tiles: every band ends inside a
+    # workgroup's sixteen tiles, the last row tile of the second is partial),
+    # at 300 in its wider form; every row against the same sequences decoded in
+    # calls of at most 64, whose products are the chunked kernel's: the same f32
+    # sums in another order
+    spec = gf.LlamaSpec(matrix_type=gf.T_Q8_0, embed_type=gf.T_Q8_0, output=False, hidden=128, intermediate=256,
+                        heads=8, kv_heads=2, vocab=vocab)
+    path = spec.write(tmp_path / "m.gguf")
+    mine = native.NativeModel(path, max_blocks=4 * nseq, block_tokens=4)
+    rng = np.random.default_rng(nseq + vocab)
+    tokens = rng.integers(0, vocab, (2, nseq))
+    a, b = ([mine.new_sequence() for _ in range(nseq)] for _ in range(2))
+    say("logits in bands", nseq, vocab)
+    for step in tokens:
+        got = mine.decode_sequences(a, [int(t) for t in step])
+        want = np.concatenate([mine.decode_sequences(b[i:i + 60], [int(t) for t in step[i:i + 60]])
+                               for i in range(0, nseq, 60)])
+        ok, err = close(got, want)
+        assert ok, (err, int(np.argmax(np.max(np.abs(got - want), axis=0))))
+
+
 def test_sequences_decode_all_or_nothing(tmp_path, ref_capi):
     spec = gf.LlamaSpec(context=12)
     path = spec.write(tmp_path / "m.gguf")

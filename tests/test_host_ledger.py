@@ -13,6 +13,8 @@
   -fsanitize=address,undefined: audited random churn, an allocation-failure
   sweep over every mutating operation (each failed call must leave the pool,
   tables and tree unchanged), and the malformed-GGUF corpus.
+* q8_pipe walks the load offsets that the tiled Q8_0 product shares with the
+  host.
 """
 
 import shutil
@@ -177,3 +179,9 @@ def test_truncate_batch_matches_single_truncations(host_lib):
     assert str(err.value) == str(err1.value)
     assert caches[0].state() == caches[1].state()
     assert caches[0].truncate_batch([], []) == 0
+
+
+def test_tiled_product_loads_stay_in_their_views(host_build):
+    # a scalar offset past a buffer view is not caught by the view's range check
+    res = subprocess.run([str(host_build / "q8_pipe")], capture_output=True, text=True, timeout=300)
+    assert res.returncode == 0 and res.stdout.startswith("passed"), res.stdout

@@ -11,6 +11,7 @@
 
 #include "model.hpp"
 #include "q8.hpp"
+#include "q8_pipe.hpp"
 #include "device_util.hpp"
 
 namespace tvara_amd {
@@ -883,8 +884,8 @@ __global__ __launch_bounds__(256) void batch_q8_kernel(const Q8BatchArgs a) {
 // Workgroups are numbered so that each XCD takes a contiguous run of tiles
 // (eight row blocks by the vector blocks), whose operands its L2 then shares.
 // Only even group counts come here (no pair is half dead).  Row tiles past the
-// matrix read zeros; vector tiles past the batch read the last tile again and
-// are not stored.
+// matrix (q8_pipe.hpp) and vector tiles past the batch read the last tile again
+// and are not stored.
 //
 // Bound: issue on the SIMDs.  At 2,048 vectors of the 16,384 x 2,048 gate|up
 // MFMAs take 43% of the cycles and the vector instructions (two thirds of them
@@ -897,7 +898,7 @@ __global__ __launch_bounds__(256) void batch_q8_kernel(const Q8BatchArgs a) {
 // the third), and 28.5 / 25.9 / 89 / 45 us at 512 against 34 / 28 / 133 / 66.
 template <int VT>
 __global__ __launch_bounds__(512, 2) void batch_q8_pipe_kernel(const Q8BatchArgs a) {
-    constexpr int BV = 2 * VT, BR = 16;  // vector and row tiles of a workgroup
+    constexpr int BV = 2 * VT, BR = kPipeRowTiles;  // vector and row tiles of a workgroup
     constexpr int XL = BV * 4 / 8;       // KiB of halves a wave loads per pair
     // separate arrays, so that the compiler sees that a step's reads do not
     // touch the buffers in flight and does not wait for them
@@ -928,19 +929,20 @@ __global__ __launch_bounds__(512, 2) void batch_q8_pipe_kernel(const Q8BatchArgs
     const __amdgpu_buffer_rsrc_t xv =
         view(a.halves, static_cast<uint32_t>(a.n_total_tiles) * static_cast<uint32_t>(a.groups) * 2048u);
     const uint32_t xoff = static_cast<uint32_t>((lane & 15) * 128 + (lane >> 4) * 16);
-    const uint32_t qoff = static_cast<uint32_t>((wave * a.pairs * 64 + lane) * 16);  // row tiles wave, wave + 8
-    const uint32_t doff = static_cast<uint32_t>((rh * 4 * a.pairs * 16 + (lane & 15)) * 4);
+    const uint32_t qoff = static_cast<uint32_t>(lane * 16), doff = static_cast<uint32_t>((lane & 15) * 4);
 
     uint4 ra[2], rb2[2];
     uint32_t da[4], db[4], dc[4];
     auto load_w = [&](int p, uint4 (&raw)[2], uint32_t (&dn)[4]) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-            raw[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                   qv, qoff, ((8 * i * a.pairs) + pbeg + p) * 1024, 0));
+        for (int i = 0; i < 2; ++i)  // row tiles wave and wave + 8 to convert
+            raw[i] = __builtin_bit_cast(
+                uint4, __builtin_amdgcn_raw_buffer_load_b128(
+                           qv, qoff, pipe_weight_offset(wave + 8 * i, tiles_here, a.pairs, pbeg + p), 0));
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-            dn[r] = __builtin_amdgcn_raw_buffer_load_b32(dv, doff, (r * a.pairs + pbeg + p) * 64, 0);
+            dn[r] = __builtin_amdgcn_raw_buffer_load_b32(
+                dv, doff, pipe_scale_offset(rh * 4 + r, tiles_here, a.pairs, pbeg + p), 0);
     };
     auto load_x = [&](int p, u32x4 (&x)[BV][4][64]) {
 #pragma unroll
