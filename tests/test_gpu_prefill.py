@@ -638,6 +638,51 @@ def test_f32_tiles(device, oracle, group, tpb, dim, fmt):
         row0 += c
 
 
+@pytest.mark.parametrize("precision", ["f32", "bf16", "f32x3"])
+def test_key_splits_of_one_long_sequence(device, oracle, precision):
+    # a few rows after a long prefix beside fresh prompts: the long rows' runs
+    # are many, the prompts' one or two, and partials exist for rows of several
+    # runs only (a slot per row and run of the longest would take 213 MB in f32
+    # and 202 MB on the bf16 tiles; these take 1 MB and 3), on a plan held open
+    # while the device's free memory is read
+    import ctypes as C
+
+    from tvara_amd import hip
+
+    heads, kv_heads, dim = 8, 2, 64
+    specs = [(16000 + 16, 16000, 16)] + [(512, 0, 512)] * 7 if precision == "f32" else \
+        [(16000 + 16, 16000, 16)] + [(300, 0, 300)] * 5
+    say("prefill splits, one long sequence", precision)
+    dev, ref, ds, rs, qs = build(device, oracle, heads, kv_heads, dim, specs, seed=140)
+    starts = [s for _, s, _ in specs]
+    counts = [r for _, _, r in specs]
+
+    def free():
+        hip.synchronize()
+        n, total = C.c_size_t(), C.c_size_t()
+        hip.check(hip.runtime().hipMemGetInfo(C.byref(n), C.byref(total)))
+        return n.value
+
+    dq, out = hip.DeviceArray.from_numpy(np.concatenate(qs)), hip.DeviceArray((sum(counts), heads * dim))
+    before = free()
+    plan = attention.PrefillPlan(dev, ds, starts, counts, heads, 1 << 20, precision)
+    used = before - free()
+    plan.launch(0, dq.ptr, out.ptr)
+    plan.check()
+    got, row0 = out.numpy(), 0
+    for q, s, st, c in zip(qs, rs, starts, counts):
+        for lo in sorted({0, 31, 32, c // 2, c - 1} & set(range(c))):
+            want = ref.fused_prompt_attention(q[lo], s, 0, st + lo, 1, heads, 1 << 20)
+            part = got[row0 + lo]
+            if precision == "bf16":
+                ok, err = bf16_ok(part, want, SHORT_ROWS)
+                assert ok, (st, lo, err)
+            else:
+                assert refmath.close(part, want, 1e-5 if precision == "f32" else TOL_F32), (st, lo)
+        row0 += c
+    assert used < 48 << 20, used
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 def test_f32_tiles_non_finite(device, dim):
     # values that are not finite reach the rows that see them and no others (a

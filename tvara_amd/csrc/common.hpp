@@ -156,11 +156,12 @@ struct PrefillArgs {
     // as DecodeArgs::kv_share: lay.kv_heads and group describe kv_share
     // virtual KV heads per KV head (GQA groups above eight)
     int kv_share;
-    // the key tiles are cut into up to `splits` runs, whose partial outputs, [split][row][heads][head_dim], and
-    // (maximum in log2 units, normaliser) pairs, [split][row][heads][2], a
-    // second kernel merges; the bf16 tiles' rows have row_splits[row] of them
-    int splits, total_rows;
-    const int* row_splits;
+    // Key splits (null: none): a row's key tiles are cut into row_runs[row].y
+    // runs.  Where they are several, run i leaves its partial output in slot
+    // row_runs[row].x + i of [slot][heads][head_dim] and its (maximum in log2
+    // units, normaliser) in [slot][heads][2], and a second kernel merges them.
+    const int2* row_runs;
+    int total_rows;
     float* part_acc;
     float* part_ml;
 };

@@ -811,35 +811,45 @@ void PrefillPlan::bf16_splits(const std::vector<int4>& seqs, int kv_heads, int p
 // XCD's L2, and each XCD's run is ordered from the most keys to the fewest
 // (MI355X, four chunks of 200-900 tokens after 500-3,000 at head_dim 128 on
 // the three-product tiles: 439 -> 261 us; even batches unchanged).
+//
+// A row's runs follow from its own chunk tile, and only rows of several leave
+// partials, each in its own slots: one long sequence beside many short ones
+// (16 rows after 16,000 tokens beside seven prompts of 512, 32 x 8 heads of 64
+// in f32) takes 4 MB of partials and 163 us, where a slot per row and run of the
+// longest took 854 MB and 425 us (row by row through the decode kernels 291 us);
+// with heads of 128 8 MB and 302 us, 1,678 MB and 855 us (518 us).  prefill_f32_shape and bf16_splits aim at 1,024 and 256 runs
+// of work, so a plan has at most twice that many workgroups with partials, of
+// 128 and 256 (row, head) pairs: 136 MB at head_dim 128.
 std::vector<int4> PrefillPlan::work_list(const std::vector<int4>& seqs, int kv_heads, int positions,
-                                         std::vector<int>& row_runs) const {
+                                         std::vector<int2>& row_runs) {
     constexpr int kXcds = 8, kCus = 32, kTileKeys = 64;
     struct Item {
         int seq, head, q0, split, tile0, end;
     };
-    std::vector<Item> items, empty;
+    std::vector<Item> items;
     int64_t total = 0;
+    slots = 0;
+    row_runs.assign(splits > 1 ? total_rows : 0, make_int2(0, 1));
     for (int i = 0; i < static_cast<int>(seqs.size()); ++i) {
         const int start = seqs[i].y, rows = seqs[i].z;
         for (int h = 0; h < kv_heads; ++h)
             for (int q0 = (rows - 1) / positions * positions; q0 >= 0; q0 -= positions) {
                 const int all = (start + std::min(q0 + positions, rows) + kTileKeys - 1) / kTileKeys;
-                if (precision == 0) {
-                    for (int s = 0; s < splits; ++s) {
-                        const int t0 = s * split_tiles, t1 = splits == 1 ? all : std::min(all, t0 + split_tiles);
-                        (t1 > t0 ? items : empty).push_back({i, h, q0, s, t0, std::max(t0, t1)});
+                int runs = splits > 1 ? (all + split_tiles - 1) / split_tiles : 1;
+                // the bf16 tiles' last run starts where every row still sees a key
+                if (precision != 0 && splits > 1) runs = std::min(runs, (start + q0) / kTileKeys / split_tiles + 1);
+                for (int s = 0; s < runs; ++s)
+                    items.push_back({i, h, q0, s, s * split_tiles, s + 1 == runs ? all : (s + 1) * split_tiles});
+                if (h == 0 && runs > 1)
+                    for (int r = seqs[i].w + q0; r < seqs[i].w + std::min(q0 + positions, rows); ++r) {
+                        row_runs[r] = make_int2(static_cast<int>(slots), runs);
+                        slots += runs;
                     }
-                } else {
-                    // the last run starts where every row still sees a key
-                    const int most = (start + q0) / kTileKeys / split_tiles + 1;
-                    const int runs = std::min({splits, (all + split_tiles - 1) / split_tiles, most});
-                    for (int s = 0; s < runs; ++s)
-                        items.push_back({i, h, q0, s, s * split_tiles, s + 1 == runs ? all : (s + 1) * split_tiles});
-                    if (splits > 1)
-                        std::fill_n(row_runs.begin() + seqs[i].w + q0, std::min(positions, rows - q0), runs);
-                }
             }
     }
+    if (!slots) row_runs.clear();
+    if (slots > static_cast<size_t>(std::numeric_limits<int>::max()))
+        throw std::invalid_argument("attention batch too large");
     for (const Item& it : items) total += it.end - it.tile0;
     // up to four rounds of the CUs, no XCD takes more workgroups than its CUs
     // need rounds for: one more would add a whole round (256 workgroups of
@@ -856,8 +866,6 @@ std::vector<int4> PrefillPlan::work_list(const std::vector<int4>& seqs, int kv_h
     }
     for (auto& r : run)
         std::stable_sort(r.begin(), r.end(), [](const Item& a, const Item& b) { return a.end - a.tile0 > b.end - b.tile0; });
-    // splits without keys write that they have none
-    for (size_t i = 0; i < empty.size(); ++i) run[i % kXcds].push_back(empty[i]);
     size_t longest = 0;
     for (const auto& r : run) longest = std::max(longest, r.size());
     if (longest * kXcds > static_cast<size_t>(std::numeric_limits<int>::max()))
@@ -942,16 +950,16 @@ void PrefillPlan::build(DeviceCache* c, const uint64_t* sequences, size_t n, siz
         throw std::invalid_argument("attention batch too large");
     const int qt = prec == 0 ? prefill_f32_positions(c->layout(), group / kv_share) : prefill_bf16_positions(group / kv_share);
     if (prec != 0) bf16_splits(sq, static_cast<int>(g.kv_heads) * kv_share, qt);
-    std::vector<int> row_runs(prec != 0 && splits > 1 ? total_rows : 0);
+    std::vector<int2> row_runs;
     std::vector<int4> list = work_list(sq, static_cast<int>(g.kv_heads) * kv_share, qt, row_runs);
     workgroups = static_cast<int>(list.size() / 2);
     runs_at = list.size();
-    list.resize(runs_at + (row_runs.size() + 3) / 4);
-    if (!row_runs.empty()) std::memcpy(list.data() + runs_at, row_runs.data(), row_runs.size() * sizeof(int));
+    list.resize(runs_at + (row_runs.size() + 1) / 2);
+    if (slots) std::memcpy(list.data() + runs_at, row_runs.data(), row_runs.size() * sizeof(int2));
     void* pt = tables.ensure(std::max<size_t>(tab.size() * sizeof(int32_t), 16));
     void* pw = work.ensure(list.size() * sizeof(int4));
     void* pe = err.ensure(sizeof(int));
-    if (splits > 1) part.ensure(static_cast<size_t>(splits) * total_rows * heads * (g.head_dim + 2) * sizeof(float));
+    if (slots) part.ensure(slots * heads * (g.head_dim + 2) * sizeof(float));
     TVARA_HIP(hipMemcpy(pt, tab.data(), tab.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     TVARA_HIP(hipMemcpy(pw, list.data(), list.size() * sizeof(int4), hipMemcpyHostToDevice));
     TVARA_HIP(hipMemset(pe, 0, sizeof(int)));
@@ -983,12 +991,11 @@ void PrefillPlan::launch(int layer, const float* q, float* out, hipStream_t s) {
     a.out = out;
     a.qscale = static_cast<float>(1.4426950408889634 / std::sqrt(static_cast<double>(cache->geometry().head_dim)));
     a.err = pinned_err ? static_cast<int*>(flag.ptr) : static_cast<int*>(err.ptr);
-    a.splits = splits;
     a.total_rows = static_cast<int>(total_rows);
-    if (splits > 1) {
-        a.row_splits = precision == 0 ? nullptr : reinterpret_cast<const int*>(a.work + runs_at);
+    if (slots) {
+        a.row_runs = reinterpret_cast<const int2*>(a.work + runs_at);
         a.part_acc = static_cast<float*>(part.ptr);
-        a.part_ml = a.part_acc + static_cast<size_t>(splits) * total_rows * heads * cache->geometry().head_dim;
+        a.part_ml = a.part_acc + slots * heads * cache->geometry().head_dim;
     }
     if (precision == 0)
         launch_prefill_f32(a, s);

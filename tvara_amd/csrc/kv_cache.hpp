@@ -270,8 +270,9 @@ struct PrefillPlan {
     bool on_rows = false;  // f32 through the decode kernels (rows_plan), not the tiles
     size_t total_rows = 0;
     AttnPlan rows_plan;
-    int splits = 1, split_tiles = 0;  // runs of key tiles per workgroup
-    size_t runs_at = 0;               // where the rows' counts of them start in `work`
+    int splits = 1, split_tiles = 0;  // the most runs of key tiles a row has, and the tiles of a run
+    size_t slots = 0;                 // partials of the rows with several runs (0: none)
+    size_t runs_at = 0;               // where the rows' first slots and runs start in `work`
     DeviceBuffer tables, work, err, part;
     // the tile kernels set the error flag in pinned host memory instead
     // (use_pinned_error: no copy back before a check)
@@ -283,9 +284,9 @@ struct PrefillPlan {
     PrefillPlan& operator=(const PrefillPlan&) = delete;
     void build(DeviceCache* c, const uint64_t* sequences, size_t count, size_t heads, size_t context,
                const size_t* start, const size_t* rows, int precision);
-    // two entries a workgroup of the tile kernels (PrefillArgs::work)
-    std::vector<int4> work_list(const std::vector<int4>& seqs, int kv_heads, int positions,
-                                std::vector<int>& row_runs) const;
+    // two entries a workgroup of the tile kernels (PrefillArgs::work); fills
+    // row_runs (PrefillArgs::row_runs, empty if no row has several) and slots
+    std::vector<int4> work_list(const std::vector<int4>& seqs, int kv_heads, int positions, std::vector<int2>& row_runs);
     // splits and split_tiles of the bf16 and three-product tiles
     void bf16_splits(const std::vector<int4>& seqs, int kv_heads, int positions);
     void use_pinned_error();

@@ -500,8 +500,9 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_bf16_kernel(const Prefill
         size_t at = static_cast<size_t>(sd.w + pos) * a.heads + head;
         float* o = a.out + at * D + 4 * g;
         float div = l;
-        if (a.splits > 1 && a.row_splits[sd.w + pos] > 1) {  // a partial
-            at += static_cast<size_t>(wk.x >> 16) * a.total_rows * a.heads;
+        const int2 runs = a.row_runs ? a.row_runs[sd.w + pos] : make_int2(0, 1);
+        if (runs.y > 1) {  // a partial
+            at = static_cast<size_t>(runs.x + (wk.x >> 16)) * a.heads + head;
             if (g == 0) *reinterpret_cast<float2*>(a.part_ml + 2 * at) = make_float2(m[nt], l);
             o = a.part_acc + at * D + 4 * g;
             bad |= !__builtin_isfinite(l);
@@ -889,7 +890,7 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_pipe_kernel(const Prefill
 template <int D, int G, int TPB>
 void launch_gt(const PrefillArgs& b, bool x3, hipStream_t s) {
     const char* env = std::getenv("TVARA_PREFILL_PIPE");
-    const bool pipe = b.splits == 1 && (env ? std::atoi(env) != 0 : D == 64);
+    const bool pipe = !b.row_runs && (env ? std::atoi(env) != 0 : D == 64);
     const bool q8 = b.lay.format == kQ8;
     constexpr int W = kWavesPerGroup;
     const dim3 grid(b.workgroups), block(64 * W);
@@ -952,7 +953,7 @@ void launch_prefill_bf16(const PrefillArgs& a, hipStream_t s, bool x3) {
         default: launch_g<8>(a, x3, s); break;
     }
     TVARA_HIP(hipGetLastError());
-    if (a.splits > 1) launch_prefill_merge(a, s);
+    if (a.row_runs) launch_prefill_merge(a, s);
 }
 
 }  // namespace tvara_amd

@@ -305,21 +305,19 @@ __global__ __launch_bounds__(64 * kRowsPerGroup / (16 * NT), 2) void prefill_f32
         }
     };
 
-    if (kt0 < ntiles) {
-        auto tile = [&](int t) { return min(t, ntiles - 1); };
-        tabload(kt0);
-        gload(kt0);
-        tabload(tile(kt0 + 1));
-        lstore(kt0, 0);
+    auto tile = [&](int t) { return min(t, ntiles - 1); };
+    tabload(kt0);
+    gload(kt0);
+    tabload(tile(kt0 + 1));
+    lstore(kt0, 0);
+    __syncthreads();
+    for (int kt = kt0; kt < ntiles; ++kt) {
+        const int buf = (kt - kt0) & 1;
+        gload(tile(kt + 1));
+        tabload(tile(kt + 2));
+        compute(kt, buf);
+        lstore(tile(kt + 1), buf ^ 1);
         __syncthreads();
-        for (int kt = kt0; kt < ntiles; ++kt) {
-            const int buf = (kt - kt0) & 1;
-            gload(tile(kt + 1));
-            tabload(tile(kt + 2));
-            compute(kt, buf);
-            lstore(tile(kt + 1), buf ^ 1);
-            __syncthreads();
-        }
     }
 
     if (__any(nonfinite != 0.f) && lane == 0) *a.err = 1;
@@ -331,10 +329,11 @@ __global__ __launch_bounds__(64 * kRowsPerGroup / (16 * NT), 2) void prefill_f32
         size_t at = static_cast<size_t>(sd.w + pos[nt]) * a.heads + head[nt];
         float* o = a.out + at * D + 16 * g;
         float inv = total;
-        if (a.splits > 1) {
-            at += static_cast<size_t>(split) * a.total_rows * a.heads;
+        const int2 runs = a.row_runs ? a.row_runs[sd.w + pos[nt]] : make_int2(0, 1);
+        if (runs.y > 1) {
+            at = static_cast<size_t>(runs.x + split) * a.heads + head[nt];
             if (g == 0) *reinterpret_cast<float2*>(a.part_ml + 2 * at) = make_float2(m[nt], total);
-            if (m[nt] == -INFINITY) continue;  // no key of this split: not read either
+            if (m[nt] == -INFINITY) continue;  // no key of this run: not used either
             o = a.part_acc + at * D + 16 * g;
             inv = 1.f;
         }
@@ -348,9 +347,10 @@ __global__ __launch_bounds__(64 * kRowsPerGroup / (16 * NT), 2) void prefill_f32
     }
 }
 
-// The splits of a (row, head) combined by log-sum-exp in split order; a
-// thread per four columns, all splits' loads of a round requested together.
-// Splits in which the row sees no key (maximum -inf) are left out.
+// The runs of a (row, head) combined by log-sum-exp in order; a thread per
+// four columns, all loads of a round of runs requested together.  Runs in which
+// the row sees no key (maximum -inf) are left out; a row of one run was written
+// by its workgroup.
 template <int D>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillArgs a) {
     constexpr int U = 8;
@@ -358,8 +358,9 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillArgs a)
     const size_t t = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x, at = t / (D / 4);
     if (at >= n) return;
     const int c = 4 * static_cast<int>(t % (D / 4));
-    const int splits = a.row_splits ? a.row_splits[at / a.heads] : a.splits;
-    if (splits == 1 && a.row_splits) return;  // written by its one workgroup
+    const int2 runs = a.row_runs[at / a.heads];
+    const int splits = runs.y;
+    if (splits == 1) return;
     float M = -INFINITY, L = 0.f;
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = 0; s0 < splits; s0 += U) {
@@ -367,7 +368,7 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillArgs a)
         f32x4 x[U];
 #pragma unroll
         for (int k = 0; k < U; ++k) {
-            const size_t p = static_cast<size_t>(min(s0 + k, splits - 1)) * n + at;
+            const size_t p = static_cast<size_t>(runs.x + min(s0 + k, splits - 1)) * a.heads + at % a.heads;
             ml[k] = *reinterpret_cast<const float2*>(a.part_ml + 2 * p);
             x[k] = *reinterpret_cast<const f32x4*>(a.part_acc + p * D + c);
         }
@@ -411,7 +412,7 @@ void launch_prefill_f32(const PrefillArgs& a, hipStream_t s) {
         launch("paged_prefill_f32", q8 ? prefill_f32_kernel<64, 2, true> : prefill_f32_kernel<64, 2, false>, grid,
                dim3(256), 0, s, a);
     TVARA_HIP(hipGetLastError());
-    if (a.splits > 1) launch_prefill_merge(a, s);
+    if (a.row_runs) launch_prefill_merge(a, s);
 }
 
 void launch_prefill_merge(const PrefillArgs& a, hipStream_t s) {
