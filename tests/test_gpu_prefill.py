@@ -684,6 +684,33 @@ def test_key_splits_of_one_long_sequence(device, oracle, precision):
 
 
 @pytest.mark.parametrize("dim", [64, 128])
+def test_f32_tiles_split_a_long_sequence_of_a_large_batch(device, oracle, dim):
+    # 1,024 workgroups and more (33 sequences of 128 rows, eight KV heads) run
+    # unsplit, unless one of them alone takes longer than a CU's share of the
+    # whole batch; whether a merge ran says which
+    heads, kv_heads = 32, 8
+    for start, merges in [(20000, 1), (0, 0)]:
+        specs = [(start + 33, start, 33)] + [(128, 0, 128)] * 33
+        say("prefill f32 large batch", dim, start)
+        dev, ref, ds, rs, qs = build(device, oracle, heads, kv_heads, dim, specs, seed=150)
+        attention.profile_enable(True)
+        attention.profile_reset()
+        try:
+            got = attention.prefill_batch(dev, np.concatenate(qs), ds, [s for _, s, _ in specs],
+                                          [r for _, _, r in specs], 0, heads, 1 << 20, precision="f32")
+            assert attention.profile_read("paged_prefill_merge")[1] == merges
+            assert attention.profile_read("paged_prefill_f32")[1] == 1
+        finally:
+            attention.profile_enable(False)
+        row0 = 0
+        for q, s, (_, st, c) in zip(qs, rs, specs):
+            for lo in (0, 31, c - 1):
+                want = ref.fused_prompt_attention(q[lo], s, 0, st + lo, 1, heads, 1 << 20)
+                assert refmath.close(got[row0 + lo], want, 1e-5), (st, lo)
+            row0 += c
+
+
+@pytest.mark.parametrize("dim", [64, 128])
 def test_f32_tiles_non_finite(device, dim):
     # values that are not finite reach the rows that see them and no others (a
     # masked probability is not multiplied by them); a key that is not finite

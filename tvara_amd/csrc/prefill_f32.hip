@@ -437,7 +437,9 @@ int prefill_f32_positions(const BlockLayout& lay, int group) {
 // 256 rows after 1,000 at 128: 72, 89, 103 in 1,024), and units of a quarter of
 // a CU's share up to 1,024 workgroups, where whole rounds of unequal
 // workgroups leave a tail (six chunks of 33-700 tokens: 328 us against 431
-// unsplit).  At least two tiles a split.
+// unsplit).  More workgroups are split so only where the longest would outlast a
+// CU's whole share: 33 rows after 130,000 tokens beside 40 prompts of 128 2,598 us row by row, 12,738 unsplit, 862 split,
+// 16 rows after 16,000 beside ten of 512 374, 1,491 and 200 (even batches of 1,024 and more are the faster unsplit).  At least two tiles a split.
 F32TileShape prefill_f32_shape(const BlockLayout& lay, int group, size_t n, const size_t* start, const size_t* rows) {
     const size_t qt = prefill_f32_positions(lay, group);
     size_t wgs = 0, work = 0, longest = 0;
@@ -456,7 +458,7 @@ F32TileShape prefill_f32_shape(const BlockLayout& lay, int group, size_t n, cons
     f.use = flops >= (lay.format == kQ8 ? 3e9 : 0.7e9);
     f.splits = 1;
     f.split_tiles = static_cast<int>(longest);
-    if (wgs < 1024) {
+    if (wgs < 1024 || longest * 256 > work) {
         const size_t units = wgs < 256 ? 256 : 1024;
         const size_t per = std::max<size_t>(2, (work + units - 1) / units);
         f.split_tiles = static_cast<int>(std::min(per, longest));
