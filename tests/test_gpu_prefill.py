@@ -683,6 +683,35 @@ def test_key_splits_of_one_long_sequence(device, oracle, precision):
     assert used < 48 << 20, used
 
 
+# (heads, KV heads, dim, format, [(prefix, rows)], tiles): few rows after long
+# prefixes, where a tile of 128 rows would be nearly empty, stay row by row
+F32_ROUTES = [(32, 8, 64, "f32", [(30000, 4)], False), (32, 8, 64, "f32", [(30000, 16)], True),
+              (32, 8, 64, "f32", [(1500, 4)] * 32, False), (32, 8, 64, "f32", [(1500, 4)] * 32 + [(0, 1500)], True),
+              (32, 8, 128, "f32", [(8000, 4)] * 2, False), (32, 8, 128, "f32", [(8000, 32)] * 2, True),
+              (9, 3, 64, "f32", [(100000, 4)], False), (9, 3, 64, "f32", [(16000, 40)], True),
+              (32, 32, 64, "f32", [(16000, 6)], False), (32, 32, 64, "f32", [(4000, 64)], True),
+              (64, 8, 128, "f32", [(8000, 1)] * 4, False), (64, 8, 128, "f32", [(8000, 8)] * 4, True),
+              (64, 8, 128, "q8_0", [(30000, 4)], False), (32, 8, 64, "q8_0", [(4000, 256)], True)]
+
+
+@pytest.mark.parametrize("heads,kv_heads,dim,fmt,chunks,tiles", F32_ROUTES)
+def test_f32_route(device, oracle, heads, kv_heads, dim, fmt, chunks, tiles):
+    specs = [(p + r, p, r) for p, r in chunks]
+    say("prefill f32 route", heads, kv_heads, dim, fmt, chunks[0], len(chunks))
+    dev, ref, ds, rs, qs = build(device, oracle, heads, kv_heads, dim, specs, seed=160, q8=fmt == "q8_0")
+    attention.profile_enable(True)
+    attention.profile_reset()
+    try:
+        got = attention.prefill_batch(dev, np.concatenate(qs), ds, [s for _, s, _ in specs], [r for _, _, r in specs],
+                                      0, heads, 1 << 20, precision="f32")
+        assert attention.profile_read("paged_prefill_f32")[1] == int(tiles)
+        assert attention.profile_read("paged_decode")[1] == int(not tiles)
+    finally:
+        attention.profile_enable(False)
+    last = ref.fused_prompt_attention(qs[-1][-1], rs[-1], 0, specs[-1][0] - 1, 1, heads, 1 << 20)
+    assert refmath.close(got.reshape(sum(len(q) for q in qs), -1)[-1], last, 1e-5)
+
+
 @pytest.mark.parametrize("dim", [64, 128])
 def test_f32_tiles_split_a_long_sequence_of_a_large_batch(device, oracle, dim):
     # 1,024 workgroups and more (33 sequences of 128 rows, eight KV heads) run

@@ -426,36 +426,54 @@ int prefill_f32_positions(const BlockLayout& lay, int group) {
     return lay.head_dim == 128 ? 8 * (16 / group) : 4 * (32 / group);
 }
 
-// Tiles or rows: a launch of tiles costs 10-12 us before its first result and
-// runs at 45-105 TFLOP/s, the decode kernels cost 5 and run at 20-40 (f32) or
-// 33-60 (Q8_0).  MI355X, tiles against rows: 25 against 26 us at 0.54 GFLOP,
-// 32 against 31.5 at 0.66, 31 against 44 at 1.0, 34 against 58 at 1.1; over
-// Q8_0 blocks 70 against 72 at 3.2 and 61 against 74 at 4.2.
+// Tiles or rows: whichever the rates below put ahead.  A tile launch costs 10 us
+// and 6.4 us of a CU per workgroup and key tile (5 where two workgroups share
+// it, at head_dim 64), for however few of its 128 rows are there.  The decode
+// kernels pay for every row, whose keys they read again, from L2: at 8 TFLOP/s
+// per query head of the group up to 26 (Q8_0 16 up to 55; 10-40 and 12-60
+// measured, as the rows' splits happen to share an XCD's L2), and at 0.7 of that
+// once a sequence's keys are past the caches.  MI355X, tiles against rows, us, 32 x
+// 8 heads of 64 in f32: one row after 130,000 tokens 421 against 106, 16 rows 429
+// against 1,233; 64 sequences after 4,000, one row each 444 against 174, 8 rows
+// 450 against 652; 8 after 16,000, 4 rows 413 against 326, 16 rows 420 against
+// 431.  Over 1,163 chunks of 1-1,000 rows in both formats the rule's choice is within
+// 0.4% of the faster one in the geometric mean and 1.41 times as long at worst,
+// always tiles 6.3% and 4.9 times.  Chunks under 0.7 GFLOP, 3 over Q8_0, are rows: tiles
+// against rows 25 against 26 us at 0.54, 32 against 31.5 at 0.66, 31 against 44
+// at 1.0; over Q8_0 70 against 72 at 3.2.
 //
 // Key splits: one workgroup per CU where the chunk alone gives fewer (64 rows
 // after 4,000 tokens, head_dim 64: 40 us in 256 units of work, 44 in 512;
 // 256 rows after 1,000 at 128: 72, 89, 103 in 1,024), and units of a quarter of
 // a CU's share up to 1,024 workgroups, where whole rounds of unequal
 // workgroups leave a tail (six chunks of 33-700 tokens: 328 us against 431
-// unsplit).  More workgroups are split so only where the longest would outlast a
-// CU's whole share: 33 rows after 130,000 tokens beside 40 prompts of 128 2,598 us row by row, 12,738 unsplit, 862 split,
-// 16 rows after 16,000 beside ten of 512 374, 1,491 and 200 (even batches of 1,024 and more are the faster unsplit).  At least two tiles a split.
+// unsplit).  At least two tiles a split.  Even batches of more workgroups are
+// faster unsplit, so they are split only where the longest would outlast a CU's
+// whole share: 33 rows after 130,000 tokens beside 40 prompts of 128 take 2,598
+// us row by row, 12,738 unsplit and 862 split, 16 after 16,000 beside ten of 512
+// 374, 1,491 and 200.
 F32TileShape prefill_f32_shape(const BlockLayout& lay, int group, size_t n, const size_t* start, const size_t* rows) {
+    const bool q8 = lay.format == kQ8;
     const size_t qt = prefill_f32_positions(lay, group);
-    size_t wgs = 0, work = 0, longest = 0;
-    double pairs = 0;  // (query, key) pairs
+    size_t wgs = 0, work = 0, read = 0, longest = 0;  // read: key tiles, as the causal mask leaves them
+    double flops = 0, row_us = 5;
+    const double rate = 1e6 * (q8 ? std::min(55, 16 * group) : std::min(26, 8 * group));  // flops per us
+    const double token_bytes = 2.0 * lay.kv_heads * lay.head_dim * (q8 ? 34.0 / 32.0 : 4.0);
     for (size_t i = 0; i < n; ++i) {
         const size_t tiles = (start[i] + rows[i] + kKeys - 1) / kKeys, w = (rows[i] + qt - 1) / qt;
         wgs += w;
         work += w * tiles;
         longest = std::max(longest, tiles);
-        pairs += static_cast<double>(rows[i]) * (start[i] + 0.5 * rows[i]);
+        for (size_t q = qt; q < rows[i] + qt; q += qt) read += (start[i] + std::min(q, rows[i]) + kKeys - 1) / kKeys;
+        const double f = 4.0 * lay.kv_heads * group * lay.head_dim * rows[i] * (start[i] + 0.5 * rows[i]);
+        flops += f;
+        row_us += f / (token_bytes * start[i] > 100e6 ? 0.7 * rate : rate);
     }
     work *= lay.kv_heads;
     wgs *= lay.kv_heads;
-    const double flops = 4.0 * lay.kv_heads * group * lay.head_dim * pairs;
+    const double tile_us = 10 + (lay.head_dim == 64 && wgs >= 256 ? 5 : 6.4) / 256 * read * lay.kv_heads;
     F32TileShape f{};
-    f.use = flops >= (lay.format == kQ8 ? 3e9 : 0.7e9);
+    f.use = flops >= (q8 ? 3e9 : 0.7e9) && tile_us < row_us;
     f.splits = 1;
     f.split_tiles = static_cast<int>(longest);
     if (wgs < 1024 || longest * 256 > work) {
