@@ -781,7 +781,10 @@ void AttnPlan::check_after(hipEvent_t after) {
 // and 314 -> 30.3 (three products), 512 after 2,000 56.3 -> 32.5, 256 after
 // 2,000 at heads of 128, three products, 168.5 -> 51.2, 900 after 1,000 over
 // Q8_0 77.2 -> 59.9.  From 256 workgroups on a split only adds rounds (256
-// of 200-260 tiles: 547 us against 770 in 512 units and 602 in 1,024).
+// of 200-260 tiles: 547 us against 770 in 512 units and 602 in 1,024), and so
+// does one that shortens the longest walk by less than a third and 16 tiles: 64
+// sequences of 40 tokens after 500 at 9 x 3 heads of 64, 192 workgroups of nine
+// tiles, 17 us against 27 in runs of seven and two.
 void PrefillPlan::bf16_splits(const std::vector<int4>& seqs, int kv_heads, int positions) {
     constexpr int64_t kUnits = 256;
     int64_t wgs = 0, total = 0;
@@ -799,6 +802,7 @@ void PrefillPlan::bf16_splits(const std::vector<int4>& seqs, int kv_heads, int p
     if (wgs >= kUnits) return;
     split_tiles = static_cast<int>(
         std::min<int64_t>(std::max<int64_t>({4, (total + kUnits - 1) / kUnits, (longest + 1023) / 1024}), longest));
+    if (3 * split_tiles > 2 * longest && longest - split_tiles < 16) split_tiles = longest;
     splits = (longest + split_tiles - 1) / split_tiles;
 }
 
