@@ -812,7 +812,9 @@ void PrefillPlan::bf16_splits(const std::vector<int4>& seqs, int kv_heads, int p
 // ragged batch, left engines idle while others held the long sequences.  So
 // the list holds only workgroups with rows, in runs of equal work per XCD that
 // keep a (sequence, KV head)'s tiles together, as they share its keys in the
-// XCD's L2, and each XCD's run is ordered from the most keys to the fewest
+// XCD's L2, and each XCD's run is ordered from the most keys to the fewest, then
+// from the most rows to the fewest (full and nearly empty chunk tiles by turns
+// would give some engines all the full ones)
 // (MI355X, four chunks of 200-900 tokens after 500-3,000 at head_dim 128 on
 // the three-product tiles: 439 -> 261 us; even batches unchanged).
 //
@@ -828,7 +830,7 @@ std::vector<int4> PrefillPlan::work_list(const std::vector<int4>& seqs, int kv_h
                                          std::vector<int2>& row_runs) {
     constexpr int kXcds = 8, kCus = 32, kTileKeys = 64;
     struct Item {
-        int seq, head, q0, split, tile0, end;
+        int seq, head, q0, rows, split, tile0, end;
     };
     std::vector<Item> items;
     int64_t total = 0;
@@ -843,7 +845,8 @@ std::vector<int4> PrefillPlan::work_list(const std::vector<int4>& seqs, int kv_h
                 // the bf16 tiles' last run starts where every row still sees a key
                 if (precision != 0 && splits > 1) runs = std::min(runs, (start + q0) / kTileKeys / split_tiles + 1);
                 for (int s = 0; s < runs; ++s)
-                    items.push_back({i, h, q0, s, s * split_tiles, s + 1 == runs ? all : (s + 1) * split_tiles});
+                    items.push_back({i, h, q0, std::min(positions, rows - q0), s, s * split_tiles,
+                                     s + 1 == runs ? all : (s + 1) * split_tiles});
                 if (h == 0 && runs > 1)
                     for (int r = seqs[i].w + q0; r < seqs[i].w + std::min(q0 + positions, rows); ++r) {
                         row_runs[r] = make_int2(static_cast<int>(slots), runs);
@@ -869,7 +872,10 @@ std::vector<int4> PrefillPlan::work_list(const std::vector<int4>& seqs, int kv_h
         before += items[i].end - items[i].tile0;
     }
     for (auto& r : run)
-        std::stable_sort(r.begin(), r.end(), [](const Item& a, const Item& b) { return a.end - a.tile0 > b.end - b.tile0; });
+        std::stable_sort(r.begin(), r.end(), [](const Item& a, const Item& b) {
+            const int ta = a.end - a.tile0, tb = b.end - b.tile0;
+            return ta != tb ? ta > tb : a.rows > b.rows;
+        });
     size_t longest = 0;
     for (const auto& r : run) longest = std::max(longest, r.size());
     if (longest * kXcds > static_cast<size_t>(std::numeric_limits<int>::max()))
