@@ -3,9 +3,11 @@
 // for every count of row tiles a workgroup can have and group pairs up to
 // those of 16,384 columns, the scalar offset lies in the view and the furthest
 // lane's read ends in it; row tiles that are there are read in their place.
+// Likewise the vectors' halves, for even and odd counts of groups.
 #include "q8_pipe.hpp"
 
 #include <cstdio>
+#include <initializer_list>
 
 using namespace tvara_amd;
 
@@ -22,6 +24,16 @@ int main() {
                     if (t < tiles) bad += w != (t * pairs + pair) * 1024 || d != (t * pairs + pair) * 64;
                     ++seen;
                 }
+    for (int groups = 1; groups <= 512; ++groups)
+        for (int tiles : {1, 2, 5, 128})
+            for (int vt = 0; vt < tiles; ++vt)
+                for (int group = 0; group < (groups + 1) / 2 * 2; ++group)
+                    for (int part = 0; part < 2; ++part) {
+                        const int x = pipe_vector_offset(vt, groups, group, part), view = tiles * groups * 2048;
+                        bad += x < 0 || x >= view || x + 15 * 128 + 3 * 16 + 16 > view;
+                        if (group < groups) bad += x != (vt * groups + group) * 2048 + part * 64;
+                        ++seen;
+                    }
     std::printf("%s: %ld loads, %ld outside their view\n", bad ? "failed" : "passed", seen, bad);
     return bad != 0;
 }

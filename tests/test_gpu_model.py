@@ -422,6 +422,35 @@ def test_prompt_passes_match_small_passes(tmp_path, name, count):
     assert ok, err
 
 
+# widths at which the products above 64 vectors run on the tiled GEMM, with even
+# and with odd counts of 32-column groups (64 and 256; 65 and 257), and row
+# counts that leave partial row tiles and workgroups
+TILED_SPECS = {
+    "even": dict(hidden=2048, intermediate=8192, heads=32, kv_heads=8),
+    "odd": dict(hidden=2080, intermediate=8224, heads=20, kv_heads=5),
+}
+
+
+@pytest.mark.parametrize("name", list(TILED_SPECS))
+def test_tiled_products_match_small_passes(tmp_path, name):
+    # prompt passes of these counts against passes of 64, whose products are the
+    # chunked kernel's: the same f32 sums of the same fp16 halves in another order
+    spec = gf.LlamaSpec(matrix_type=gf.T_Q8_0, context=2200, layers=1, **TILED_SPECS[name])
+    path = spec.write(tmp_path / "m.gguf")
+    mine = native.NativeModel(path, max_blocks=4 * (2200 // 16) + 8, block_tokens=16)
+    for count in (65, 96, 130, 257, 300, 511, 2047):
+        tokens = [int(t) for t in np.random.default_rng(count).integers(0, spec.vocab, count)]
+        seq, small = mine.new_sequence(), mine.new_sequence()
+        got = mine.prefill(seq, tokens)
+        for lo in range(0, count, 64):
+            want = mine.prefill(small, tokens[lo:lo + 64])
+        ok, err = close(got, want)
+        say("tiled products", name, count, "relative logit difference", err)
+        assert ok, (count, err)
+        mine.drop_sequence(seq)
+        mine.drop_sequence(small)
+
+
 def test_prefill_matches_reference_last_logits(tmp_path, ref_capi):
     # tvara_sequence_prefill: the last token's logits of a chunked pass, with
     # decode_batch's checks, messages and rollback

@@ -883,9 +883,10 @@ __global__ __launch_bounds__(256) void batch_q8_kernel(const Q8BatchArgs a) {
 // waves a SIMD.
 // Workgroups are numbered so that each XCD takes a contiguous run of tiles
 // (eight row blocks by the vector blocks), whose operands its L2 then shares.
-// Only even group counts come here (no pair is half dead).  Row tiles past the
-// matrix (q8_pipe.hpp) and vector tiles past the batch read the last tile again
-// and are not stored.
+// Row tiles past the matrix and vector tiles past the batch read the last tile
+// again and are not stored; the group that completes an odd count has weights
+// and scales of zero (as the matrix was laid out) and multiplies the last one's
+// halves (q8_pipe.hpp).
 //
 // Bound: issue on the SIMDs.  At 2,048 vectors of the 16,384 x 2,048 gate|up
 // MFMAs take 43% of the cycles and the vector instructions (two thirds of them
@@ -950,7 +951,8 @@ __global__ __launch_bounds__(512, 2) void batch_q8_pipe_kernel(const Q8BatchArgs
             const int t = (wave * XL + i) / 4, part = (wave * XL + i) % 4;
             const int vt = min(vb * BV + t, a.n_total_tiles - 1);
             __builtin_amdgcn_raw_ptr_buffer_load_lds(xv, (__attribute__((address_space(3))) void*)&x[t][part][0], 16, xoff,
-                                                     (vt * a.groups + 2 * (pbeg + p) + part / 2) * 2048 + part % 2 * 64, 0, 0);
+                                                     pipe_vector_offset(vt, a.groups, 2 * (pbeg + p) + part / 2, part % 2), 0,
+                                                     0);
         }
     };
     auto stage = [&](const uint4 (&raw)[2], half8 (&ws)[2][BR][64]) {
@@ -1471,7 +1473,7 @@ PipePlan pipe_plan(const Weight& w, int n, int tiles, int most_splits = 8) {
 // launch that reads the weights again (MI355X, a layer's four products: 79 us
 // against 87 at 96 vectors, 81 against 93 at 128); at 64 the chunked kernel
 // takes 45 us, this one 67.
-bool pipe_for(const Weight& w, int n) { return w.q8 && w.groups() % 2 == 0 && n > 64; }
+bool pipe_for(const Weight& w, int n) { return w.q8 && n > 64; }
 
 // row tiles [tile0, tile1), K in `per` groups a split
 void launch_pipe(const Weight& w, const PipePlan& p, int tile0, int tile1, const _Float16* halves,

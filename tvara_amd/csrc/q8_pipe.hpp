@@ -1,8 +1,8 @@
-// Where the tiled Q8_0 product (batch_q8_pipe_kernel) reads its weights:
-// plain arithmetic, shared with a host test that walks every shape.
+// Where the tiled Q8_0 product (batch_q8_pipe_kernel) reads its weights and
+// vectors: plain arithmetic, shared with a host test that walks every shape.
 //
-// The kernel's buffer views cover one workgroup's row tiles, and a load's tile
-// is part of its scalar offset.  A raw buffer load compares its vector offset
+// The kernel's buffer views cover one workgroup's row tiles, and all vectors; a
+// load's tile is part of its scalar offset.  A raw buffer load compares its vector offset
 // with what the view has left after the scalar one, which says nothing once
 // the scalar offset is past the view; so a scalar offset always lies in it:
 // row tiles past the matrix read its last one again, and their rows are not
@@ -24,6 +24,12 @@ constexpr int pipe_weight_offset(int t, int tiles, int pairs, int pair) {
 }
 constexpr int pipe_scale_offset(int t, int tiles, int pairs, int pair) {
     return (pipe_row_tile(t, tiles) * pairs + pair) * kQ8PairScales;
+}
+
+// scalar offset of the halves (part 0: hi, 1: lo) of a group of vector tile vt,
+// which must exist; lane l adds 128 bytes times l%16 and 16 times l/16
+constexpr int pipe_vector_offset(int vt, int groups, int group, int part) {
+    return (vt * groups + (group < groups ? group : groups - 1)) * 2048 + part * 64;
 }
 
 }  // namespace tvara_amd
