@@ -234,23 +234,23 @@ def test_sequences_decode_matches_serial_reference(tmp_path, ref_capi, nseq, emb
     say("sequences_decode", nseq, "worst relative logit error", worst)
 
 
-@pytest.mark.parametrize("vocab", [32800, 34001])
+@pytest.mark.parametrize("hidden,vocab", [(1024, 32700), (128, 34001)])
 @pytest.mark.parametrize("nseq", [65, 130, 300])
-def test_many_sequences_logits_in_bands(tmp_path, nseq, vocab):
-    # above 64 sequences the logits are the tiled product's, computed in four
-    # bands of row tiles (2,050 and 2,126 tiles: every band ends inside a
-    # workgroup's sixteen tiles, the last row tile of the second is partial),
-    # at 300 in its wider form; every row against the same sequences decoded in
-    # calls of at most 64, whose products are the chunked kernel's: the same f32
-    # sums in another order
-    spec = gf.LlamaSpec(matrix_type=gf.T_Q8_0, embed_type=gf.T_Q8_0, output=False, hidden=128, intermediate=256,
+def test_many_sequences_logits_in_bands(tmp_path, nseq, hidden, vocab):
+    # the logits of more than 64 sequences, computed in four bands of row tiles:
+    # by the tiled product at hidden 1,024 (2,044 tiles: every band ends inside a
+    # workgroup's sixteen tiles, the last row tile is partial), by the chunked
+    # kernel in several blocks of vectors at 128 (300: tiled too); every row
+    # against the same sequences decoded in calls of at most 64, one block of the
+    # chunked kernel: the same f32 sums in another order
+    spec = gf.LlamaSpec(matrix_type=gf.T_Q8_0, embed_type=gf.T_Q8_0, output=False, hidden=hidden, intermediate=256,
                         heads=8, kv_heads=2, vocab=vocab)
     path = spec.write(tmp_path / "m.gguf")
     mine = native.NativeModel(path, max_blocks=4 * nseq, block_tokens=4)
     rng = np.random.default_rng(nseq + vocab)
     tokens = rng.integers(0, vocab, (2, nseq))
     a, b = ([mine.new_sequence() for _ in range(nseq)] for _ in range(2))
-    say("logits in bands", nseq, vocab)
+    say("logits in bands", nseq, hidden, vocab)
     for step in tokens:
         got = mine.decode_sequences(a, [int(t) for t in step])
         want = np.concatenate([mine.decode_sequences(b[i:i + 60], [int(t) for t in step[i:i + 60]])
@@ -405,10 +405,11 @@ def test_chunk_tiles_beyond_fp16_take_the_rows(tmp_path, monkeypatch):
 @pytest.mark.parametrize("count", [65, 128, 129, 256, 257, 2047, 2100])
 @pytest.mark.parametrize("name", ["q8_0-d64", "q8_0-d64-g16"])
 def test_prompt_passes_match_small_passes(tmp_path, name, count):
-    # the tiled products of a prompt pass (above 64 vectors; above 256 in the
-    # wider tile; a second pass after 2,048 tokens) against passes of 64, whose
-    # products stream the weights: the same f32 sums of the same fp16 halves in
-    # another order, so within a few rounding steps of sums over 1,024 columns
+    # the products of a prompt pass above 64 vectors (small matrices: the chunked
+    # kernel in several blocks of vectors, tiled ones at 2,047; a second pass
+    # after 2,048 tokens) against passes of 64: the same f32 sums of the same fp16
+    # halves in another order, so within a few rounding steps of sums over 1,024
+    # columns
     spec = gf.LlamaSpec(**{**CHUNK_SPECS[name], "context": 2200, "layers": 2})
     path = spec.write(tmp_path / "m.gguf")
     tokens = [int(t) for t in np.random.default_rng(count).integers(0, spec.vocab, count)]

@@ -185,3 +185,18 @@ def test_tiled_product_loads_stay_in_their_views(host_build):
     # a scalar offset past a buffer view is not caught by the view's range check
     res = subprocess.run([str(host_build / "q8_pipe")], capture_output=True, text=True, timeout=300)
     assert res.returncode == 0 and res.stdout.startswith("passed"), res.stdout
+
+
+# rows, columns, vectors, kernel (0: chunked, else the tiled one's vector tiles a
+# wave): small matrices stay on the chunked kernel, whose workgroups are small,
+# and the shapes of tests/test_gpu_model.py run on what they are there for
+PRODUCTS = [(960, 576, 128, 0), (3072, 576, 512, 0), (3072, 576, 2048, 4), (2048, 2048, 128, 0), (2048, 2048, 512, 2),
+            (16384, 2048, 65, 2), (16384, 2048, 512, 4), (16448, 2080, 65, 4), (16448, 2080, 300, 4),
+            (2080, 8224, 257, 2), (2080, 8224, 2047, 4), (32700, 1024, 65, 2), (32700, 1024, 300, 2),
+            (34001, 128, 65, 0), (34001, 128, 130, 0), (128256, 2048, 64, 0), (128256, 2048, 65, 4)]
+
+
+@pytest.mark.parametrize("rows,cols,n,kernel", PRODUCTS)
+def test_product_kernel(host_build, rows, cols, n, kernel):
+    args = [str(host_build / "q8_pipe"), "choice", str((rows + 15) // 16), str(cols // 32), str(n)]
+    assert int(subprocess.run(args, capture_output=True, text=True, check=True).stdout) == kernel

@@ -695,11 +695,10 @@ struct Q8BatchArgs {
     const float* unscale;
     int rows, tiles, groups, pairs;  // tiles: one past the last row tile of this launch
     int tile0;                       // its first row tile (blockIdx.x counts from it)
-    int n, vt0;                      // vectors in this launch, first vector tile
-    int n_total;
+    int n;              // vectors
     int n_total_tiles;  // vector tiles the halves hold
     int groups_per_split;
-    float* out;  // [gridDim.y][n_total][rows]
+    float* out;  // [gridDim.y][n][rows]
 };
 
 // A workgroup of NT waves covers RT row tiles (RT x 16 rows) over a share of
@@ -751,7 +750,8 @@ __global__ __launch_bounds__(256) void batch_q8_kernel(const Q8BatchArgs a) {
     const __amdgpu_buffer_rsrc_t dv = view(reinterpret_cast<const uint32_t*>(a.d) + static_cast<size_t>(t0) * a.pairs * 16,
                                            static_cast<uint32_t>(tiles_here * a.pairs) * 64u);
     const uint32_t xbytes = static_cast<uint32_t>(a.groups) * 2048u;
-    const __amdgpu_buffer_rsrc_t xv = view(a.halves + static_cast<size_t>(a.vt0 + wave) * a.groups * 2 * 64, xbytes);
+    const int vt = min(static_cast<int>(blockIdx.z) * NT + wave, a.n_total_tiles - 1);  // (past the batch: not stored)
+    const __amdgpu_buffer_rsrc_t xv = view(a.halves + static_cast<size_t>(vt) * a.groups * 2 * 64, xbytes);
     // byte offsets of this thread's load slots within a chunk
     uint32_t qoff[WPT], doff[DPT];
 #pragma unroll
@@ -855,12 +855,11 @@ __global__ __launch_bounds__(256) void batch_q8_kernel(const Q8BatchArgs a) {
         load_x(min(k + 3, nchunks - 1), xB);
     }
     // lane l holds row l%16 of each tile for vectors 4(l/16) + i of its tile
-    float* out = a.out + static_cast<size_t>(blockIdx.y) * a.n_total * a.rows;
+    float* out = a.out + static_cast<size_t>(blockIdx.y) * a.n * a.rows;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int jl = wave * 16 + 4 * (lane >> 4) + i;
-        if (jl >= a.n) continue;
-        const int j = a.vt0 * 16 + jl;
+        const int j = (static_cast<int>(blockIdx.z) * NT + wave) * 16 + 4 * (lane >> 4) + i;
+        if (j >= a.n) continue;
         const float us = a.unscale[j];
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
@@ -1033,7 +1032,7 @@ __global__ __launch_bounds__(512, 2) void batch_q8_pipe_kernel(const Q8BatchArgs
     // no load may be in flight into this workgroup's LDS when it ends
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // lane l holds row l%16 of each row tile for vectors 4(l/16) + i
-    float* out = a.out + static_cast<size_t>(blockIdx.y) * a.n_total * a.rows;
+    float* out = a.out + static_cast<size_t>(blockIdx.y) * a.n * a.rows;
 #pragma unroll
     for (int v = 0; v < VT; ++v)
 #pragma unroll
@@ -1417,26 +1416,6 @@ void launch_batch_q8(int nt, dim3 grid, hipStream_t s, const Q8BatchArgs& a) {
     }
 }
 
-// row tiles per workgroup and groups per K split of the batched Q8_0
-// product: four row tiles from 1,024 tiles up, else two (more workgroups for
-// the smaller matrices); the groups are split while the launch has fewer than
-// 512 workgroups (two per CU), in whole chunks of four groups, never below
-// eight groups and into at most eight splits (the epilogues read every split)
-struct Q8Plan {
-    int rt, gx, per, splits;
-};
-Q8Plan q8_plan(const Weight& w) {
-    Q8Plan p{};
-    const int tiles = w.tiles(), groups = w.groups();
-    p.rt = tiles >= 1024 ? 4 : 2;
-    p.gx = (tiles + p.rt - 1) / p.rt;
-    const int want = p.gx >= 512 ? 1 : std::min({(512 + p.gx - 1) / p.gx, std::max(1, groups / 8), 8});
-    p.per = (groups + want - 1) / want;
-    p.per = (p.per + 3) / 4 * 4;  // whole chunks, so splits start on a group pair
-    p.splits = (groups + p.per - 1) / p.per;
-    return p;
-}
-
 struct F32Plan {
     int tiles, per, splits;
 };
@@ -1450,34 +1429,11 @@ F32Plan f32_plan(int rows, int cols) {
     return p;
 }
 
-// Plan of the tiled GEMM: VT = 4 (128 vectors a workgroup) above 256 vectors,
-// else 2, and K split while the launch has fewer than 256 workgroups (one a
-// CU), into at most eight splits of at least eight groups.  MI355X, the four
-// products of a Llama-3.2-1B layer together: VT = 2 takes 110 us at 256
-// vectors, 173 at 384 and 200 at 512, VT = 4 129, 167 and 180.
-struct PipePlan {
-    int vt, gx, per, splits;  // vector tiles a wave, workgroups per split, groups per split, splits
-};
-PipePlan pipe_plan(const Weight& w, int n, int tiles, int most_splits = 8) {
-    PipePlan p{};
-    const int vtiles = (n + 15) / 16;
-    p.vt = n > 256 ? 4 : 2;
-    p.gx = ((tiles + 15) / 16) * ((vtiles + 2 * p.vt - 1) / (2 * p.vt));
-    const int want = std::min({std::max(1, 256 / p.gx), std::max(1, w.groups() / 8), most_splits});
-    p.per = ((w.groups() + want - 1) / want + 1) / 2 * 2;  // whole pairs
-    p.splits = (w.groups() + p.per - 1) / p.per;
-    return p;
-}
-
-// The tiled GEMM above 64 vectors, where the chunked kernel needs a second
-// launch that reads the weights again (MI355X, a layer's four products: 79 us
-// against 87 at 96 vectors, 81 against 93 at 128); at 64 the chunked kernel
-// takes 45 us, this one 67.
-bool pipe_for(const Weight& w, int n) { return w.q8 && n > 64; }
+int pipe_for(const Weight& w, int n) { return w.q8 ? pipe_choice(w.tiles(), w.groups(), n) : 0; }
 
 // row tiles [tile0, tile1), K in `per` groups a split
-void launch_pipe(const Weight& w, const PipePlan& p, int tile0, int tile1, const _Float16* halves,
-                 const float* unscale, int n, float* out, hipStream_t s) {
+Q8BatchArgs batch_args(const Weight& w, int per, int tile0, int tile1, const _Float16* halves, const float* unscale,
+                       int n, float* out) {
     Q8BatchArgs a{};
     a.q = static_cast<const uint4*>(w.q.ptr);
     a.d = static_cast<const uint16_t*>(w.d.ptr);
@@ -1489,10 +1445,27 @@ void launch_pipe(const Weight& w, const PipePlan& p, int tile0, int tile1, const
     a.groups = w.groups();
     a.pairs = w.pairs();
     a.n = n;
-    a.n_total = n;
     a.n_total_tiles = (n + 15) / 16;
-    a.groups_per_split = p.per;
+    a.groups_per_split = per;
     a.out = out;
+    return a;
+}
+
+// the chunked kernel over every block of up to four vector tiles
+void launch_chunked(const Weight& w, int rt, int splits, int per, int tile0, int tile1, const _Float16* halves,
+                    const float* unscale, int n, float* out, hipStream_t s) {
+    const Q8BatchArgs a = batch_args(w, per, tile0, tile1, halves, unscale, n, out);
+    const int nt = std::min(4, a.n_total_tiles);
+    const dim3 grid((tile1 - tile0 + rt - 1) / rt, splits, (a.n_total_tiles + 3) / 4);
+    if (rt == 4)
+        launch_batch_q8<4>(nt, grid, s, a);
+    else
+        launch_batch_q8<2>(nt, grid, s, a);
+}
+
+void launch_pipe(const Weight& w, const PipePlan& p, int tile0, int tile1, const _Float16* halves,
+                 const float* unscale, int n, float* out, hipStream_t s) {
+    const Q8BatchArgs a = batch_args(w, p.per, tile0, tile1, halves, unscale, n, out);
     if (static_cast<double>(a.n_total_tiles) * a.groups * 2048 >= 2147483648.0)
         throw std::invalid_argument("batched product input above 2 GiB");
     const dim3 grid(p.gx, p.splits);
@@ -1503,11 +1476,12 @@ void launch_pipe(const Weight& w, const PipePlan& p, int tile0, int tile1, const
 }
 }  // namespace
 
-bool halves_by_line(const Weight& w, int n) { return pipe_for(w, n); }
+bool halves_by_line(const Weight& w, int n) { return pipe_for(w, n) != 0; }
 
 int batch_splits(const Weight& w, int n) {
     if (!w.q8) return f32_plan(w.rows, w.cols).splits;
-    return pipe_for(w, n) ? pipe_plan(w, n, w.tiles()).splits : q8_plan(w).splits;
+    const int vt = pipe_for(w, n);
+    return vt ? pipe_plan(w.tiles(), w.groups(), n, vt).splits : q8_plan(w.tiles(), w.groups()).splits;
 }
 
 size_t batch_part_floats(const Weight& w, int n) {
@@ -1520,32 +1494,11 @@ size_t batch_part_floats(const Weight& w, int n) {
 
 void launch_batch_product(const Weight& w, const float* x, const _Float16* halves, const float* unscale, int n,
                           float* out, hipStream_t s) {
-    if (pipe_for(w, n)) {
-        launch_pipe(w, pipe_plan(w, n, w.tiles()), 0, w.tiles(), halves, unscale, n, out, s);
+    if (const int vt = pipe_for(w, n)) {
+        launch_pipe(w, pipe_plan(w.tiles(), w.groups(), n, vt), 0, w.tiles(), halves, unscale, n, out, s);
     } else if (w.q8) {
-        const Q8Plan p = q8_plan(w);
-        for (int j0 = 0; j0 < n; j0 += 64) {
-            const int nj = std::min(64, n - j0);
-            Q8BatchArgs a{};
-            a.q = static_cast<const uint4*>(w.q.ptr);
-            a.d = static_cast<const uint16_t*>(w.d.ptr);
-            a.halves = reinterpret_cast<const uint4*>(halves);
-            a.unscale = unscale;
-            a.rows = w.rows;
-            a.tiles = w.tiles();
-            a.groups = w.groups();
-            a.pairs = w.pairs();
-            a.n = nj;
-            a.vt0 = j0 / 16;
-            a.n_total = n;
-            a.groups_per_split = p.per;
-            a.out = out;
-            const dim3 grid(p.gx, p.splits);
-            if (p.rt == 4)
-                launch_batch_q8<4>((nj + 15) / 16, grid, s, a);
-            else
-                launch_batch_q8<2>((nj + 15) / 16, grid, s, a);
-        }
+        const Q8Plan p = q8_plan(w.tiles(), w.groups());
+        launch_chunked(w, p.rt, p.splits, p.per, 0, w.tiles(), halves, unscale, n, out, s);
     } else {
         if (w.cols % kTileK) throw std::invalid_argument("batched matvec needs a row width divisible by 32");
         const F32Plan p = f32_plan(w.rows, w.cols);
@@ -1570,35 +1523,13 @@ void launch_batch_product_tiles(const Weight& w, int tile0, int tile1, const _Fl
                                 int n, float* out, hipStream_t s) {
     if (!w.q8 || batch_splits(w, n) != 1 || tile0 < 0 || tile0 >= tile1 || tile1 > w.tiles())
         throw std::invalid_argument("row-tile range of a batched product needs an unsplit Q8_0 matrix");
-    if (pipe_for(w, n)) {
-        launch_pipe(w, pipe_plan(w, n, tile1 - tile0, 1), tile0, tile1, halves, unscale, n, out, s);
+    if (const int vt = pipe_for(w, n)) {
+        launch_pipe(w, pipe_plan(tile1 - tile0, w.groups(), n, vt, 1), tile0, tile1, halves, unscale, n, out, s);
         TVARA_HIP(hipGetLastError());
         return;
     }
-    const Q8Plan p = q8_plan(w);
-    for (int j0 = 0; j0 < n; j0 += 64) {
-        const int nj = std::min(64, n - j0);
-        Q8BatchArgs a{};
-        a.q = static_cast<const uint4*>(w.q.ptr);
-        a.d = static_cast<const uint16_t*>(w.d.ptr);
-        a.halves = reinterpret_cast<const uint4*>(halves);
-        a.unscale = unscale;
-        a.rows = w.rows;
-        a.tiles = tile1;
-        a.tile0 = tile0;
-        a.groups = w.groups();
-        a.pairs = w.pairs();
-        a.n = nj;
-        a.vt0 = j0 / 16;
-        a.n_total = n;
-        a.groups_per_split = p.per;
-        a.out = out;
-        const dim3 grid((tile1 - tile0 + p.rt - 1) / p.rt, 1);
-        if (p.rt == 4)
-            launch_batch_q8<4>((nj + 15) / 16, grid, s, a);
-        else
-            launch_batch_q8<2>((nj + 15) / 16, grid, s, a);
-    }
+    const Q8Plan p = q8_plan(w.tiles(), w.groups());
+    launch_chunked(w, p.rt, 1, p.per, tile0, tile1, halves, unscale, n, out, s);
     TVARA_HIP(hipGetLastError());
 }
 
