@@ -259,6 +259,23 @@ def test_many_sequences_logits_in_bands(tmp_path, nseq, hidden, vocab):
         assert ok, (err, int(np.argmax(np.max(np.abs(got - want), axis=0))))
 
 
+@pytest.mark.parametrize("vocab", [20000, 140000])
+def test_tokens_match_prompt_pass(tmp_path, vocab):
+    # the token's products of a model whose weights fit the memory-side cache and
+    # of one (300 MB) whose weights pass through it, against the batched ones
+    spec = gf.LlamaSpec(matrix_type=gf.T_Q8_0, embed_type=gf.T_Q8_0, output=False, hidden=2048, intermediate=512,
+                        layers=1, heads=32, kv_heads=8, vocab=vocab)
+    path = spec.write(tmp_path / "m.gguf")
+    mine = native.NativeModel(path, max_blocks=32, block_tokens=16)
+    tokens = [int(t) for t in np.random.default_rng(vocab).integers(0, vocab, 20)]
+    a, b = mine.new_sequence(), mine.new_sequence()
+    for t in tokens:
+        got = mine.logits(a, t)
+    ok, err = close(got, mine.prefill(b, tokens))
+    say("token by token", vocab, "relative logit difference", err)
+    assert ok, err
+
+
 def test_sequences_decode_all_or_nothing(tmp_path, ref_capi):
     spec = gf.LlamaSpec(context=12)
     path = spec.write(tmp_path / "m.gguf")

@@ -143,6 +143,11 @@ DeviceModel::DeviceModel(const std::string& path, size_t max_blocks, size_t bloc
         load_weight({{p + "ffn_gate.weight", I}, {p + "ffn_up.weight", I}}, H, L.gate_up, true);
         load_weight({{p + "ffn_down.weight", H}}, I, L.down);
     }
+    size_t read = (has_output_ ? output_ : embedding_).bytes();  // by every token
+    for (const Layer& L : layers_) read += L.qkv.bytes() + L.out.bytes() + L.gate_up.bytes() + L.down.bytes();
+    const bool streamed = read > kMemoryCacheBytes;
+    embedding_.streamed = output_.streamed = streamed;
+    for (Layer& L : layers_) L.qkv.streamed = L.out.streamed = L.gate_up.streamed = L.down.streamed = streamed;
     int bad = 0;
     TVARA_HIP(hipMemcpy(&bad, bad_.ptr, sizeof(int), hipMemcpyDeviceToHost));
     if (bad) throw std::invalid_argument("nonfinite model weight");

@@ -23,6 +23,8 @@ struct MatvecSegment {
     const float* residual;
 };
 
+constexpr size_t kMemoryCacheBytes = size_t(256) << 20;  // MI355X, behind the XCDs' L2s
+
 // A weight matrix in HBM: f32 rows, or Q8_0 kept quantised.  The Q8_0 form
 // is tiled for the kernels that read it: rows are cut into tiles of 16
 // (zero-padded) and the groups of 32 columns into pairs (an odd last group
@@ -41,6 +43,10 @@ struct Weight {
     // a fused gate|up block stored with its rows interleaved (row 2i is gate
     // row i, 2i + 1 is up row i), so that the SwiGLU pairs meet in a tile
     bool interleaved = false;
+    // the model's weights outgrow the memory-side cache, so that nothing is left
+    // of them by the next token (matvec_q8_kernel)
+    bool streamed = false;
+    size_t bytes() const { return f32.bytes + q.bytes + d.bytes; }
     int tiles() const { return (rows + 15) / 16; }
     int groups() const { return cols / 32; }
     int pairs() const { return (groups() + 1) / 2; }

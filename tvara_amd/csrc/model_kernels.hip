@@ -406,7 +406,7 @@ __device__ __forceinline__ void write_segment(const MatvecSegment* seg, int nseg
 // once.  Pairs past the share, and the zero group that completes an odd
 // count, are selected away rather than multiplied (their loads stay in
 // bounds).
-template <int W, int RT>
+template <int W, int RT, bool kStream>
 __global__ __launch_bounds__(W * 64) void matvec_q8_kernel(const Q8MatvecArgs a) {
     constexpr int U = 2;
     extern __shared__ float vs[];  // cols floats
@@ -420,11 +420,15 @@ __global__ __launch_bounds__(W * 64) void matvec_q8_kernel(const Q8MatvecArgs a)
     for (int r = 0; r < RT; ++r) tl[r] = min(static_cast<int>(blockIdx.x) * RT + r, a.tiles - 1);
     // U pairs of every tile from pair p on, clamped to the wave's last pair
     // (a wave without pairs reads pair P - 1 and adds nothing).  The weights
-    // are read once a token and pass through L2 non-temporally, or each layer's
-    // 65 MB would evict the next kernels' code and inputs from it (Llama-3.2-1B,
-    // one token: the layers' attention kernel 13.2 -> 10.7 us, the call 850 ->
+    // are read once a token.  Those of a model that outgrows the 256 MB
+    // memory-side cache pass through the caches non-temporally, or each layer's
+    // 65 MB would evict the next kernels' code and inputs (Llama-3.2-1B, one
+    // token: the layers' attention kernel 13.2 -> 10.7 us, the call 850 ->
     // 799; their scales, half a line a read, stay cached: streamed too, the
-    // gate|up product takes 12.3 against 11.9 us).
+    // gate|up product takes 12.3 against 11.9 us).  A smaller model's are still
+    // there at the next token and stay.  Kernel time a token, kept against
+    // streamed: SmolLM2-135M's shape, 143 MB, 747 against 800 us; three layers of
+    // TinyLlama's, 200 MB, 119 against 125; six, 335 MB, 239 against 235.
     auto load = [&](int p, uint4 (&qq)[RT][U], uint32_t (&dd)[RT][U]) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -432,8 +436,8 @@ __global__ __launch_bounds__(W * 64) void matvec_q8_kernel(const Q8MatvecArgs a)
 #pragma unroll
             for (int r = 0; r < RT; ++r) {
                 const size_t blk = static_cast<size_t>(tl[r]) * P + pc;
-                qq[r][u] = __builtin_bit_cast(
-                    uint4, __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(a.q) + blk * 64 + lane));
+                const u32x4* at = reinterpret_cast<const u32x4*>(a.q) + blk * 64 + lane;
+                qq[r][u] = __builtin_bit_cast(uint4, kStream ? __builtin_nontemporal_load(at) : *at);
                 dd[r][u] = a.d[blk * 16 + (lane & 15)];
             }
         }
@@ -1388,18 +1392,20 @@ void launch_matvec_q8(const Weight& w, const float* v, const MatvecSegment* seg,
     const dim3 grid(wgs);
     // the input, and the norm weights beside it when the product normalises
     const size_t lds = static_cast<size_t>(w.cols) * sizeof(float) * (norm_w ? 2 : 1);
-    auto go = [&](auto kernel, int waves) { launch("model_matvec_q8", kernel, grid, dim3(64 * waves), lds, s, a); };
+    auto go = [&](auto kernel, auto streaming, int waves) {
+        launch("model_matvec_q8", w.streamed ? streaming : kernel, grid, dim3(64 * waves), lds, s, a);
+    };
     if (rt == 2) {
-        if (want >= 8) go(matvec_q8_kernel<8, 2>, 8);
-        else if (want >= 4) go(matvec_q8_kernel<4, 2>, 4);
-        else if (want >= 2) go(matvec_q8_kernel<2, 2>, 2);
-        else go(matvec_q8_kernel<1, 2>, 1);
+        if (want >= 8) go(matvec_q8_kernel<8, 2, false>, matvec_q8_kernel<8, 2, true>, 8);
+        else if (want >= 4) go(matvec_q8_kernel<4, 2, false>, matvec_q8_kernel<4, 2, true>, 4);
+        else if (want >= 2) go(matvec_q8_kernel<2, 2, false>, matvec_q8_kernel<2, 2, true>, 2);
+        else go(matvec_q8_kernel<1, 2, false>, matvec_q8_kernel<1, 2, true>, 1);
     } else {
-        if (want >= 16) go(matvec_q8_kernel<16, 1>, 16);
-        else if (want >= 8) go(matvec_q8_kernel<8, 1>, 8);
-        else if (want >= 4) go(matvec_q8_kernel<4, 1>, 4);
-        else if (want >= 2) go(matvec_q8_kernel<2, 1>, 2);
-        else go(matvec_q8_kernel<1, 1>, 1);
+        if (want >= 16) go(matvec_q8_kernel<16, 1, false>, matvec_q8_kernel<16, 1, true>, 16);
+        else if (want >= 8) go(matvec_q8_kernel<8, 1, false>, matvec_q8_kernel<8, 1, true>, 8);
+        else if (want >= 4) go(matvec_q8_kernel<4, 1, false>, matvec_q8_kernel<4, 1, true>, 4);
+        else if (want >= 2) go(matvec_q8_kernel<2, 1, false>, matvec_q8_kernel<2, 1, true>, 2);
+        else go(matvec_q8_kernel<1, 1, false>, matvec_q8_kernel<1, 1, true>, 1);
     }
     TVARA_HIP(hipGetLastError());
 }
