@@ -798,3 +798,50 @@ def test_tile_key_splits(device, oracle, group, tpb, dim, fmt, precision):
         assert ok, err
     else:
         assert refmath.close(got, want, TOL_F32), refmath.max_rel(got, want)
+
+
+@pytest.mark.parametrize("precision", ["bf16", "f32x3"])
+@pytest.mark.parametrize("dim", [64, 128])
+def test_tile_key_splits_reject_what_unsplit_tiles_reject(device, dim, precision):
+    # a chunk whose keys run as splits: a value that is not finite (seen by rows
+    # of one split only), a key or query outside the fp16 range in three
+    # products, and values whose weighted sum overflows f32 only once the splits
+    # are added (equal scores: every weight is 1, and 4,000 of 2e35 pass f32's
+    # largest while the 256 of a split stay below); the largest sum that fits
+    # goes through
+    heads, kv_heads, n, rows = 8, 2, 4000, 40
+    w = kv_heads * dim
+    k, v = (synth.normal(7, t, n * w).reshape(n, w) for t in "kv")
+    q = synth.normal(7, "q", rows * heads * dim).reshape(rows, -1)
+
+    def run(k, v, q):
+        c = device.PagedCache(1, kv_heads, dim, 16, n // 16 + 4)
+        s = c.create_sequence()
+        c.append_many(s, k, v)
+        return attention.prefill_batch(c, q, [s], [n - rows], [rows], 0, heads, 1 << 20, precision=precision)
+
+    say("prefill split rejections", dim, precision)
+    assert np.isfinite(run(k, v, q)).all()
+    for at in (5, n - 20):
+        bad = v.copy()
+        bad[at, 3] = np.nan
+        with pytest.raises(device.InvalidArgument):
+            run(k, bad, q)
+        bad = k.copy()
+        bad[at, 3] = np.inf
+        with pytest.raises(device.InvalidArgument):
+            run(bad, v, q)
+        if precision == "f32x3":
+            bad[at, 3] = 7e4
+            with pytest.raises(device.InvalidArgument):
+                run(bad, v, q)
+    if precision == "f32x3":
+        bad = q.copy()
+        bad[rows - 1, 2] = -1e6
+        with pytest.raises(device.InvalidArgument):
+            run(k, v, bad)
+    zero = np.zeros_like(q)
+    with pytest.raises(device.InvalidArgument):
+        run(k, np.full_like(v, 2e35), zero)
+    got = run(k, np.full_like(v, 2e34), zero)
+    assert refmath.close(got / 2e34, np.ones_like(got), 1e-2)

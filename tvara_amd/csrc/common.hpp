@@ -211,7 +211,8 @@ bool prefill_bf16_supported(const BlockLayout& lay, int group);
 bool prefill_x3_supported(const BlockLayout& lay, int group);
 void launch_prefill_bf16(const PrefillArgs& a, hipStream_t s, bool x3 = false);
 int prefill_bf16_positions(int group);  // chunk positions of a workgroup
-// the splits of a row combined into a.out (prefill_f32.hip)
+// the splits of a row combined into a.out; a result that is not finite sets
+// *a.err unless that is null (prefill_f32.hip)
 void launch_prefill_merge(const PrefillArgs& a, hipStream_t s);
 // prefill_f32.hip: the same layouts in f32
 void launch_prefill_f32(const PrefillArgs& a, hipStream_t s);

@@ -390,7 +390,12 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillArgs a)
         }
         M = mc;
     }
-    *reinterpret_cast<f32x4*>(a.out + at * D + c) = sum / L;
+    const f32x4 out = sum / L;
+    // (a.err null: the f32 tiles, whose values may be anything)
+    if (a.err && !(__builtin_isfinite(out[0]) && __builtin_isfinite(out[1]) && __builtin_isfinite(out[2]) &&
+                   __builtin_isfinite(out[3])))
+        *a.err = 1;
+    *reinterpret_cast<f32x4*>(a.out + at * D + c) = out;
 }
 
 }  // namespace
@@ -412,7 +417,11 @@ void launch_prefill_f32(const PrefillArgs& a, hipStream_t s) {
         launch("paged_prefill_f32", q8 ? prefill_f32_kernel<64, 2, true> : prefill_f32_kernel<64, 2, false>, grid,
                dim3(256), 0, s, a);
     TVARA_HIP(hipGetLastError());
-    if (a.row_runs) launch_prefill_merge(a, s);
+    if (a.row_runs) {
+        PrefillArgs m = a;
+        m.err = nullptr;
+        launch_prefill_merge(m, s);
+    }
 }
 
 void launch_prefill_merge(const PrefillArgs& a, hipStream_t s) {
