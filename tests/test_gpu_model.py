@@ -21,8 +21,8 @@ from pathlib import Path
 import numpy as np
 import pytest
 
+from tvara_amd import attention, native
 from tvara_amd import gguf_writer as gf
-from tvara_amd import native
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-4
@@ -417,6 +417,34 @@ def test_chunk_tiles_beyond_fp16_take_the_rows(tmp_path, monkeypatch):
         mine.close()
     assert np.isfinite(got["rows"]).all()
     assert np.array_equal(got["tiles"], got["rows"])
+
+
+def test_prompt_tiles_beyond_fp16_take_the_rows(tmp_path, monkeypatch):
+    # the same in a prompt longer than the rows' passes of 512: the pass of 1,300
+    # on the tiles is run again in the passes that the rows take by themselves
+    spec = gf.LlamaSpec(**{**CHUNK_SPECS["f32-d128"], "context": 1400}, attn_norm_scale=2e5)
+    path = spec.write(tmp_path / "m.gguf")
+    tokens = [int(t) for t in np.random.default_rng(9).integers(0, spec.vocab, 1300)]
+    got = {}
+    for choice in ("tiles", "rows"):
+        monkeypatch.setenv("TVARA_CHUNK_ATTENTION", choice)
+        mine = native.NativeModel(path, max_blocks=100, block_tokens=16)
+        sm = mine.new_sequence()
+        attention.profile_enable(True)
+        attention.profile_reset()
+        try:
+            got[choice] = mine.prefill(sm, tokens)
+            # three passes of at most 512 rows in each of two layers
+            assert attention.profile_read("paged_decode")[1] == 6
+            assert attention.profile_read("paged_prefill_x3")[1] == (2 if choice == "tiles" else 0)
+        finally:
+            attention.profile_enable(False)
+        assert mine.cache().length(sm) == len(tokens)
+        got[choice + " next"] = mine.logits(sm, 3)
+        mine.close()
+    assert np.isfinite(got["rows"]).all()
+    assert np.array_equal(got["tiles"], got["rows"])
+    assert np.array_equal(got["tiles next"], got["rows next"])
 
 
 @pytest.mark.parametrize("count", [65, 128, 129, 256, 257, 2047, 2100])

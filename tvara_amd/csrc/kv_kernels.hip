@@ -119,15 +119,16 @@ __global__ __launch_bounds__(kThreads) void append_rows_f32_kernel(char* pool, B
 }
 
 // One layer's rows of reserved tokens (DeviceCache::reserve_tokens): grid.x =
-// op, grid.y = kind; source rows are [src_row][kv_width].  Plain stores: the
-// attention of the same layer reads them next.
+// op, grid.y = kind; source rows are [op][kv_width], so that any run of the
+// reserved tokens can be written by itself.  Plain stores: the attention of the
+// same layer reads them next.
 __global__ __launch_bounds__(kThreads) void write_layer_rows_kernel(char* pool, BlockLayout lay,
                                                                     const RowOp* __restrict__ ops, int layer,
                                                                     const float* __restrict__ keys,
                                                                     const float* __restrict__ values) {
     const RowOp op = ops[blockIdx.x];
     const int kind = blockIdx.y;
-    const float* src = (kind ? values : keys) + static_cast<size_t>(op.src_row) * lay.kv_width;
+    const float* src = (kind ? values : keys) + static_cast<size_t>(blockIdx.x) * lay.kv_width;
     float* dst = reinterpret_cast<float*>(pool + static_cast<size_t>(op.block) * lay.stride) +
                  (static_cast<size_t>(layer * 2 + kind) * lay.tpb + op.slot) * lay.kv_width;
     if ((lay.kv_width & 3) == 0) {

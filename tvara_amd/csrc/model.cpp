@@ -526,43 +526,42 @@ void DeviceModel::decode_chunk(uint64_t sequence, const uint32_t* tokens, size_t
     hipStream_t s = cache_->stream();
     const int heads = static_cast<int>(c.heads);
     std::vector<size_t> positions(rows);
-    std::vector<uint64_t> seq_of_row(rows, sequence);
     for (size_t c0 = 0; c0 < n; c0 += rows) {
-        const size_t m = std::min(rows, n - c0);
-        positions.resize(m);
-        seq_of_row.resize(m);
-        for (size_t j = 0; j < m; ++j) positions[j] = position + c0 + j;
-        stage_rows(tokens + c0, positions.data(), m);
+        const size_t chunk = std::min(rows, n - c0);
         // the chunk's tokens join the sequence now (their blocks zero-filled or
         // copied on write); every layer writes its K/V rows into their slots
         // before its attention reads them
-        const RowOp* slots = cache_->reserve_tokens(sequence, m);
-        const bool last = c0 + m == n, logits = !(last_only && !last);
-        const size_t out_rows = last_only ? 1 : m;
-        // One pass over the layers, the logits and their copy.  A pass on the
-        // tiles returns false when their flag is raised: a query or key beyond
-        // the fp16 range (or a non-finite input); the chunk is then staged
-        // again and takes the f32 rows, which rewrite the same slots.
-        auto pass = [&](bool on_tiles) {
+        const RowOp* slots = cache_->reserve_tokens(sequence, chunk);
+        // One pass of m of the chunk's tokens from r0 over the layers, the logits
+        // and their copy.  A pass on the tiles takes the whole chunk and returns
+        // false when their flag is raised: a query or key beyond the fp16 range
+        // (or a non-finite input); the chunk is then staged again and takes the f32
+        // rows, which rewrite the same slots, kChunkRows at a time.
+        auto pass = [&](bool on_tiles, size_t r0, size_t m) {
+            const bool last = c0 + r0 + m == n, logits = !(last_only && !last);
+            const size_t out_rows = last_only ? 1 : m;
+            positions.resize(m);
+            for (size_t j = 0; j < m; ++j) positions[j] = position + c0 + r0 + j;
+            stage_rows(tokens + c0 + r0, positions.data(), m);
             // row j sees the cached tokens and the chunk up to itself
             // (fused_prompt_attention, attention.hpp:85-89)
             std::function<void(hipEvent_t)> check;
             Attend attend;
             if (on_tiles) {
-                const size_t start = position + c0;
+                const size_t start = position + c0 + r0;
                 chunk_plan_.build(cache_.get(), &sequence, 1, c.heads, c.context, &start, &m, 2);
                 chunk_plan_.use_pinned_error();
                 attend = [&](int l, const float* q, float* kl, float* vl, float* attn) {
-                    cache_->write_layer_rows(slots, m, l, kl, vl);
+                    cache_->write_layer_rows(slots + r0, m, l, kl, vl);
                     chunk_plan_.launch(l, q, attn, s);
                 };
                 check = [&](hipEvent_t e) { chunk_plan_.check_after(e); };
             } else {
                 std::vector<size_t> lengths(m);
                 for (size_t j = 0; j < m; ++j) lengths[j] = positions[j] + 1;
-                batch_plan_.build(cache_.get(), seq_of_row, lengths, {}, heads, 0);
+                batch_plan_.build(cache_.get(), std::vector<uint64_t>(m, sequence), lengths, {}, heads, 0);
                 attend = [&](int l, const float* q, float* kl, float* vl, float* attn) {
-                    cache_->write_layer_rows(slots, m, l, kl, vl);
+                    cache_->write_layer_rows(slots + r0, m, l, kl, vl);
                     batch_plan_.launch(l, q, nullptr, nullptr, attn, s);
                 };
                 check = [&](hipEvent_t e) { batch_plan_.check_after(e); };
@@ -580,13 +579,11 @@ void DeviceModel::decode_chunk(uint64_t sequence, const uint32_t* tokens, size_t
             } else {
                 check(step_events_.attn);
             }
-            if (logits) copy_logits(bands, out_rows, last_only ? logits_host : logits_host + c0 * c.vocab);
+            if (logits) copy_logits(bands, out_rows, last_only ? logits_host : logits_host + (c0 + r0) * c.vocab);
             return true;
         };
-        if (!pass(tiles)) {
-            stage_rows(tokens + c0, positions.data(), m);
-            pass(false);
-        }
+        if (!tiles || !pass(true, 0, chunk))
+            for (size_t r0 = 0; r0 < chunk; r0 += kChunkRows) pass(false, r0, std::min(kChunkRows, chunk - r0));
     }
 }
 
