@@ -13,8 +13,9 @@
   -fsanitize=address,undefined: audited random churn, an allocation-failure
   sweep over every mutating operation (each failed call must leave the pool,
   tables and tree unchanged), and the malformed-GGUF corpus.
-* q8_pipe walks the load offsets that the tiled Q8_0 product shares with the
-  host.
+* q8_pipe walks the plans and load offsets of the batched Q8_0 products;
+  plan_pool runs the pool of closed plans' buffers on a stand-in for HIP's
+  runtime.
 """
 
 import shutil
@@ -200,3 +201,8 @@ PRODUCTS = [(960, 576, 128, 0), (3072, 576, 512, 0), (3072, 576, 2048, 4), (2048
 def test_product_kernel(host_build, rows, cols, n, kernel):
     args = [str(host_build / "q8_pipe"), "choice", str((rows + 15) // 16), str(cols // 32), str(n)]
     assert int(subprocess.run(args, capture_output=True, text=True, check=True).stdout) == kernel
+
+
+def test_plan_pool(host_build):
+    res = subprocess.run([str(host_build / "plan_pool")], capture_output=True, text=True, timeout=300)
+    assert res.returncode == 0 and res.stdout == "passed\n", res.stdout + res.stderr[-3000:]

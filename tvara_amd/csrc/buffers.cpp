@@ -1,0 +1,110 @@
+// Device and pinned host buffers, and the plan pool (see buffers.hpp).
+#include "buffers.hpp"
+
+#include <algorithm>
+
+namespace tvara_amd {
+
+namespace {
+size_t pages(size_t n) { return (n + 4095) / 4096 * 4096; }
+}  // namespace
+
+void* DeviceBuffer::ensure(size_t n) {
+    if (n <= bytes && ptr) return ptr;
+    if (ptr) {
+        TVARA_HIP(hipDeviceSynchronize());
+        TVARA_HIP(hipFree(ptr));
+        ptr = nullptr;
+        bytes = 0;
+    }
+    const size_t want = std::max<size_t>(pages(n), 4096);
+    TVARA_HIP(hipMalloc(&ptr, want));
+    bytes = want;
+    return ptr;
+}
+
+DeviceBuffer::~DeviceBuffer() {
+    if (ptr) (void)hipFree(ptr);
+}
+
+void* PinnedBuffer::acquire(size_t n) {
+    if (done) TVARA_HIP(hipEventSynchronize(done));
+    if (n > bytes || !ptr) {
+        if (ptr) TVARA_HIP(hipHostFree(ptr));
+        ptr = nullptr;
+        const size_t want = std::max<size_t>(pages(n), 4096);
+        TVARA_HIP(hipHostMalloc(&ptr, want, hipHostMallocDefault));
+        bytes = want;
+    }
+    return ptr;
+}
+
+void PinnedBuffer::release(hipStream_t s) {
+    if (!done) TVARA_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
+    TVARA_HIP(hipEventRecord(done, s));
+}
+
+PinnedBuffer::~PinnedBuffer() {
+    if (done) {
+        (void)hipEventSynchronize(done);
+        (void)hipEventDestroy(done);
+    }
+    if (ptr) (void)hipHostFree(ptr);
+}
+
+PlanPool::Set::~Set() {
+    if (idle) (void)hipEventDestroy(idle);
+}
+
+std::unique_ptr<PlanPool::Set> PlanPool::take(size_t bytes) {
+    int device = 0;
+    TVARA_HIP(hipGetDevice(&device));
+    std::unique_ptr<Set> out;
+    {
+        std::lock_guard<std::mutex> hold(lock_);
+        size_t best = sets_.size();
+        for (size_t i = 0; i < sets_.size(); ++i)
+            if (sets_[i]->device == device && sets_[i]->region.bytes >= bytes &&
+                (best == sets_.size() || sets_[i]->region.bytes < sets_[best]->region.bytes) &&
+                hipEventQuery(sets_[i]->idle) == hipSuccess)
+                best = i;
+        (void)hipGetLastError();  // (not ready is no error)
+        if (best < sets_.size()) {
+            out = std::move(sets_[best]);
+            sets_.erase(sets_.begin() + static_cast<std::ptrdiff_t>(best));
+        }
+    }
+    if (!out) {
+        // the event is made here, where the plan's device is the current one: a
+        // plan may be closed with another one current
+        out = std::make_unique<Set>();
+        out->device = device;
+        TVARA_HIP(hipEventCreateWithFlags(&out->idle, hipEventDisableTiming));
+    }
+    return out;
+}
+
+void PlanPool::give(std::unique_ptr<Set> s) {
+    int device = -1;
+    if (s->region.bytes <= kSetBytes && s->idle && hipGetDevice(&device) == hipSuccess && device == s->device &&
+        hipEventRecord(s->idle, nullptr) == hipSuccess) {
+        std::lock_guard<std::mutex> hold(lock_);
+        if (!closed_) {
+            sets_.push_back(std::move(s));
+            if (sets_.size() > kSets) {
+                s = std::move(sets_.front());  // the oldest goes
+                sets_.erase(sets_.begin());
+            }
+        }
+    }
+    // what is left in s is freed here, outside the lock (hipFree waits for its work)
+}
+
+void PlanPool::close() {
+    std::vector<std::unique_ptr<Set>> rest;
+    std::lock_guard<std::mutex> hold(lock_);
+    closed_ = true;
+    rest.swap(sets_);
+}
+
+}  // namespace tvara_amd

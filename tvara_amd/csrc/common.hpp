@@ -9,14 +9,10 @@
 #include <stdexcept>
 #include <string>
 
+#include "hip_check.hpp"
 #include "kv_ledger.hpp"
 
 namespace tvara_amd {
-
-inline void hip_check(hipError_t e, const char* what) {
-    if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
-}
-#define TVARA_HIP(x) ::tvara_amd::hip_check((x), #x)
 
 enum Format : int { kF32 = 0, kQ8 = 1 };
 

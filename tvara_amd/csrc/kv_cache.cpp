@@ -22,51 +22,6 @@ size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 enum Slot { kInitOps = 0, kRowOps = 1, kKeys = 2, kValues = 3, kMisc = 4, kMiscOut = 5 };
 }  // namespace
 
-// -------------------------------------------------------------- buffers
-
-void* DeviceBuffer::ensure(size_t n) {
-    if (n <= bytes && ptr) return ptr;
-    if (ptr) {
-        TVARA_HIP(hipDeviceSynchronize());
-        TVARA_HIP(hipFree(ptr));
-        ptr = nullptr;
-        bytes = 0;
-    }
-    const size_t want = std::max<size_t>(round_up(n, 4096), 4096);
-    TVARA_HIP(hipMalloc(&ptr, want));
-    bytes = want;
-    return ptr;
-}
-
-DeviceBuffer::~DeviceBuffer() {
-    if (ptr) (void)hipFree(ptr);
-}
-
-void* PinnedBuffer::acquire(size_t n) {
-    if (done) TVARA_HIP(hipEventSynchronize(done));
-    if (n > bytes || !ptr) {
-        if (ptr) TVARA_HIP(hipHostFree(ptr));
-        ptr = nullptr;
-        const size_t want = std::max<size_t>(round_up(n, 4096), 4096);
-        TVARA_HIP(hipHostMalloc(&ptr, want, hipHostMallocDefault));
-        bytes = want;
-    }
-    return ptr;
-}
-
-void PinnedBuffer::release(hipStream_t s) {
-    if (!done) TVARA_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
-    TVARA_HIP(hipEventRecord(done, s));
-}
-
-PinnedBuffer::~PinnedBuffer() {
-    if (done) {
-        (void)hipEventSynchronize(done);
-        (void)hipEventDestroy(done);
-    }
-    if (ptr) (void)hipHostFree(ptr);
-}
-
 // host vector -> device scratch slot, through pinned memory, on the stream
 template <class T>
 static T* upload(DeviceCache& c, int slot, const T* data, size_t count) {
@@ -573,52 +528,6 @@ void AttnPlan::place() {
     char* host = static_cast<char*>(buf->staging.acquire(copied));
     place_in(device, buf->region.bytes, s, host);
     buf->staging.release(s);
-}
-
-PlanPool::Set::~Set() {
-    if (idle) (void)hipEventDestroy(idle);
-}
-
-std::unique_ptr<PlanPool::Set> PlanPool::take(size_t bytes) {
-    std::unique_ptr<Set> out;
-    {
-        std::lock_guard<std::mutex> hold(lock_);
-        size_t best = sets_.size();
-        for (size_t i = 0; i < sets_.size(); ++i)
-            if (sets_[i]->region.bytes >= bytes && (best == sets_.size() || sets_[i]->region.bytes < sets_[best]->region.bytes) &&
-                hipEventQuery(sets_[i]->idle) == hipSuccess)
-                best = i;
-        (void)hipGetLastError();  // (not ready is no error)
-        if (best < sets_.size()) {
-            out = std::move(sets_[best]);
-            sets_.erase(sets_.begin() + static_cast<std::ptrdiff_t>(best));
-        }
-    }
-    return out ? std::move(out) : std::make_unique<Set>();
-}
-
-void PlanPool::give(std::unique_ptr<Set> s) {
-    // (an event of another device than the current one fails to record)
-    if (s->region.bytes <= kSetBytes &&
-        (s->idle || hipEventCreateWithFlags(&s->idle, hipEventDisableTiming) == hipSuccess) &&
-        hipEventRecord(s->idle, nullptr) == hipSuccess) {
-        std::lock_guard<std::mutex> hold(lock_);
-        if (!closed_) {
-            sets_.push_back(std::move(s));
-            if (sets_.size() > kSets) {
-                s = std::move(sets_.front());  // the oldest goes
-                sets_.erase(sets_.begin());
-            }
-        }
-    }
-    // what is left in s is freed here, outside the lock (hipFree waits for its work)
-}
-
-void PlanPool::close() {
-    std::vector<std::unique_ptr<Set>> rest;
-    std::lock_guard<std::mutex> hold(lock_);
-    closed_ = true;
-    rest.swap(sets_);
 }
 
 namespace {

@@ -8,60 +8,12 @@
 #include <cstdint>
 #include <map>
 #include <memory>
-#include <mutex>
 #include <vector>
 
+#include "buffers.hpp"
 #include "common.hpp"
 
 namespace tvara_amd {
-
-// Grow-only device buffer.
-struct DeviceBuffer {
-    void* ptr = nullptr;
-    size_t bytes = 0;
-    void* ensure(size_t n);
-    ~DeviceBuffer();
-};
-
-// Grow-only pinned host buffer whose reuse waits for the last copy out of it.
-struct PinnedBuffer {
-    void* ptr = nullptr;
-    size_t bytes = 0;
-    hipEvent_t done = nullptr;
-    void* acquire(size_t n);
-    void release(hipStream_t s);
-    ~PinnedBuffer();
-};
-
-// Buffers of closed decode plans, kept by a cache for its next plans: a
-// serving loop makes a plan per step, and allocating and freeing its device
-// region and pinned memory, which waits for the device, cost it a quarter of the
-// step (MI355X, 32 sequences, 16 layers: 518 -> 379 us with the append).  A set
-// is handed out only after the event recorded behind its last plan's work, so
-// neither a launch nor a late error flag of the old plan can meet the new one.
-// Only plans whose every launch went to the null stream come here: it outlives
-// any plan and is never captured.  At most kSets sets of at most kSetBytes;
-// the rest is freed as before.  The cache frees the sets when it goes; plans
-// may outlive it.
-class PlanPool {
-public:
-    struct Set {
-        DeviceBuffer region;
-        PinnedBuffer staging, flag;
-        hipEvent_t idle = nullptr;
-        ~Set();
-    };
-    // a set whose region holds `bytes` and whose work has ended, or a new one
-    std::unique_ptr<Set> take(size_t bytes);
-    void give(std::unique_ptr<Set> s);
-    void close();
-
-private:
-    static constexpr size_t kSets = 4, kSetBytes = size_t(64) << 20;
-    std::mutex lock_;
-    std::vector<std::unique_ptr<Set>> sets_;
-    bool closed_ = false;
-};
 
 class DeviceCache {
 public:
