@@ -22,6 +22,7 @@ hipError_t result(hipError_t e) {
     if (e != hipSuccess) last = e;
     return e;
 }
+hipError_t query_result = hipSuccess;
 size_t held(int d) {
     size_t n = 0;
     for (const auto& m : memory)
@@ -59,6 +60,7 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
 }
 hipError_t hipEventQuery(hipEvent_t e) {
     auto* ev = reinterpret_cast<Event*>(e);
+    if (query_result != hipSuccess) return result(query_result);
     return result(ev->recorded && !ev->ended ? hipErrorNotReady : hipSuccess);
 }
 hipError_t hipEventSynchronize(hipEvent_t e) { return reinterpret_cast<Event*>(e)->ended = true, hipSuccess; }
@@ -130,11 +132,41 @@ void devices() {
     pool.close();
     last = hipSuccess;
 }
+
+// what the pool does is not seen in the last error, and what others left there
+// is not lost
+void errors() {
+    PlanPool pool;
+    pool.give(made(pool, 10000));
+    made(pool, 10000);
+    check(last == hipSuccess, "an event that is not ready is no error");
+    end_all();
+    last = hipErrorLaunchFailure;
+    made(pool, 10000);
+    check(last == hipErrorLaunchFailure, "an earlier error stays for its check");
+    last = hipSuccess;
+    query_result = hipErrorLaunchFailure;
+    made(pool, 10000);
+    check(last == hipErrorLaunchFailure, "a query's own error stays for the next check");
+    query_result = last = hipSuccess;
+    auto s = made(pool, 10000);
+    record_result = hipErrorStreamCaptureImplicit;
+    const size_t before = memory.size();
+    pool.give(std::move(s));
+    check(memory.size() == before - 1 && last == hipSuccess, "a record that fails frees the set and is no error");
+    s = made(pool, 20000);
+    last = hipErrorLaunchFailure;
+    pool.give(std::move(s));
+    check(last != hipSuccess, "an earlier error stays beside it");
+    record_result = last = hipSuccess;
+    pool.close();
+}
 }  // namespace
 
 int main() {
     reuse();
     devices();
+    errors();
     std::printf("%s\n", failures ? "failed" : "passed");
     return failures != 0;
 }

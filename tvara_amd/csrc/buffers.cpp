@@ -60,15 +60,20 @@ std::unique_ptr<PlanPool::Set> PlanPool::take(size_t bytes) {
     int device = 0;
     TVARA_HIP(hipGetDevice(&device));
     std::unique_ptr<Set> out;
-    {
+    // An event that is not ready leaves that as the runtime's last error, which
+    // is cleared; an error that waits there already, or any other answer of a
+    // query, is for the caller's next check.
+    if (hipPeekAtLastError() == hipSuccess) {
         std::lock_guard<std::mutex> hold(lock_);
         size_t best = sets_.size();
-        for (size_t i = 0; i < sets_.size(); ++i)
-            if (sets_[i]->device == device && sets_[i]->region.bytes >= bytes &&
-                (best == sets_.size() || sets_[i]->region.bytes < sets_[best]->region.bytes) &&
-                hipEventQuery(sets_[i]->idle) == hipSuccess)
-                best = i;
-        (void)hipGetLastError();  // (not ready is no error)
+        for (size_t i = 0; i < sets_.size(); ++i) {
+            if (sets_[i]->device != device || sets_[i]->region.bytes < bytes ||
+                (best < sets_.size() && sets_[i]->region.bytes >= sets_[best]->region.bytes))
+                continue;
+            const hipError_t e = hipEventQuery(sets_[i]->idle);
+            if (e == hipSuccess) best = i;
+            if (e == hipErrorNotReady) (void)hipGetLastError();
+        }
         if (best < sets_.size()) {
             out = std::move(sets_[best]);
             sets_.erase(sets_.begin() + static_cast<std::ptrdiff_t>(best));
@@ -86,8 +91,15 @@ std::unique_ptr<PlanPool::Set> PlanPool::take(size_t bytes) {
 
 void PlanPool::give(std::unique_ptr<Set> s) {
     int device = -1;
-    if (s->region.bytes <= kSetBytes && s->idle && hipGetDevice(&device) == hipSuccess && device == s->device &&
-        hipEventRecord(s->idle, nullptr) == hipSuccess) {
+    bool marked = s->region.bytes <= kSetBytes && s->idle && hipGetDevice(&device) == hipSuccess && device == s->device;
+    if (marked) {
+        // a record that fails (a stream that the null stream waits for is being
+        // captured, say) only means that the set is freed: no later check's error
+        const bool clean = hipPeekAtLastError() == hipSuccess;
+        marked = hipEventRecord(s->idle, nullptr) == hipSuccess;
+        if (!marked && clean) (void)hipGetLastError();
+    }
+    if (marked) {
         std::lock_guard<std::mutex> hold(lock_);
         if (!closed_) {
             sets_.push_back(std::move(s));
