@@ -161,12 +161,34 @@ void errors() {
     record_result = last = hipSuccess;
     pool.close();
 }
+
+// at most four sets and 64 MiB stay, the latest ones; one above that does not
+void bounds() {
+    PlanPool pool;
+    std::unique_ptr<PlanPool::Set> s[6];
+    for (auto& x : s) x = made(pool, 10000);
+    for (auto& x : s) pool.give(std::move(x));
+    check(memory.size() == 4, "four sets stay");
+    pool.clear();
+    check(memory.empty() && events.empty(), "a cleared pool holds nothing");
+    constexpr size_t MiB = size_t(1) << 20;
+    for (int i = 0; i < 4; ++i) s[i] = made(pool, 20 * MiB);
+    for (int i = 0; i < 4; ++i) pool.give(std::move(s[i]));
+    check(held(0) == 60 * MiB, "64 MiB stay at most");
+    pool.give(made(pool, 64 * MiB));
+    check(held(0) == 64 * MiB, "the latest stays");
+    pool.give(made(pool, 65 * MiB));
+    check(held(0) == 64 * MiB, "a set above the bound does not come in");
+    pool.close();
+    check(memory.empty() && events.empty(), "a closed pool holds nothing");
+}
 }  // namespace
 
 int main() {
     reuse();
     devices();
     errors();
+    bounds();
     std::printf("%s\n", failures ? "failed" : "passed");
     return failures != 0;
 }

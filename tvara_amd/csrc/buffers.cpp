@@ -2,6 +2,7 @@
 #include "buffers.hpp"
 
 #include <algorithm>
+#include <array>
 
 namespace tvara_amd {
 
@@ -89,9 +90,9 @@ std::unique_ptr<PlanPool::Set> PlanPool::take(size_t bytes) {
     return out;
 }
 
-void PlanPool::give(std::unique_ptr<Set> s) {
+void PlanPool::give(std::unique_ptr<Set> s) noexcept {
     int device = -1;
-    bool marked = s->region.bytes <= kSetBytes && s->idle && hipGetDevice(&device) == hipSuccess && device == s->device;
+    bool marked = s->region.bytes <= kBytes && s->idle && hipGetDevice(&device) == hipSuccess && device == s->device;
     if (marked) {
         // a record that fails (a stream that the null stream waits for is being
         // captured, say) only means that the set is freed: no later check's error
@@ -99,24 +100,35 @@ void PlanPool::give(std::unique_ptr<Set> s) {
         marked = hipEventRecord(s->idle, nullptr) == hipSuccess;
         if (!marked && clean) (void)hipGetLastError();
     }
+    std::array<std::unique_ptr<Set>, kSets + 1> gone;  // freed outside the lock (hipFree waits for a set's work)
     if (marked) {
         std::lock_guard<std::mutex> hold(lock_);
         if (!closed_) {
             sets_.push_back(std::move(s));
-            if (sets_.size() > kSets) {
-                s = std::move(sets_.front());  // the oldest goes
+            size_t bytes = 0;
+            for (const auto& k : sets_) bytes += k->region.bytes;
+            for (size_t i = 0; sets_.size() > kSets || bytes > kBytes; ++i) {
+                bytes -= sets_.front()->region.bytes;
+                gone[i] = std::move(sets_.front());
                 sets_.erase(sets_.begin());
             }
         }
     }
-    // what is left in s is freed here, outside the lock (hipFree waits for its work)
+}
+
+void PlanPool::clear() {
+    std::array<std::unique_ptr<Set>, kSets> gone;
+    std::lock_guard<std::mutex> hold(lock_);
+    std::move(sets_.begin(), sets_.end(), gone.begin());
+    sets_.clear();
 }
 
 void PlanPool::close() {
-    std::vector<std::unique_ptr<Set>> rest;
-    std::lock_guard<std::mutex> hold(lock_);
-    closed_ = true;
-    rest.swap(sets_);
+    {
+        std::lock_guard<std::mutex> hold(lock_);
+        closed_ = true;
+    }
+    clear();
 }
 
 }  // namespace tvara_amd

@@ -36,8 +36,9 @@ struct PinnedBuffer {
 // neither a launch nor a late error flag of the old plan can meet the new one.
 // Only plans whose every launch went to the null stream come here: it outlives
 // any plan and is never captured; only on the device that they were allocated
-// on.  At most kSets sets of at most kSetBytes; the rest is freed as before.  The cache frees the sets when it goes; plans
-// may outlive it.
+// on.  At most kSets sets of at most kBytes together; the oldest are freed.  The
+// cache frees the sets when it goes (plans may outlive it), and when a plan finds
+// no device memory.
 class PlanPool {
 public:
     struct Set {
@@ -49,13 +50,15 @@ public:
     };
     // a set whose region holds `bytes` and whose work has ended, or a new one
     std::unique_ptr<Set> take(size_t bytes);
-    void give(std::unique_ptr<Set> s);
-    void close();
+    void give(std::unique_ptr<Set> s) noexcept;
+    void clear();  // frees the sets that are here
+    void close();  // and keeps none from now on
+    PlanPool() { sets_.reserve(kSets + 1); }  // give() allocates nothing: it runs in destructors
 
 private:
-    static constexpr size_t kSets = 4, kSetBytes = size_t(64) << 20;
+    static constexpr size_t kSets = 4, kBytes = size_t(64) << 20;
     std::mutex lock_;
-    std::vector<std::unique_ptr<Set>> sets_;
+    std::vector<std::unique_ptr<Set>> sets_;  // oldest first
     bool closed_ = false;
 };
 

@@ -524,7 +524,14 @@ void AttnPlan::place() {
         home = cache->plan_pool();
         buf = s ? std::make_unique<PlanPool::Set>() : home->take(total);
     }
-    char* device = static_cast<char*>(buf->region.ensure(total));
+    char* device;
+    try {
+        device = static_cast<char*>(buf->region.ensure(total));
+    } catch (const std::runtime_error&) {  // no memory, unless closed plans hold some
+        (void)hipGetLastError();
+        cache->plan_pool()->clear();
+        device = static_cast<char*>(buf->region.ensure(total));
+    }
     char* host = static_cast<char*>(buf->staging.acquire(copied));
     place_in(device, buf->region.bytes, s, host);
     buf->staging.release(s);
