@@ -609,6 +609,39 @@ def test_pipelined_kernel_ragged_chunks(device, oracle, monkeypatch, group, tpb)
     assert ok, err
 
 
+@pytest.mark.parametrize("fmt", ["f32", "q8_0"])
+@pytest.mark.parametrize("tpb", [16, 32, 64, 128])
+def test_pipelined_kernel_over_blocks(device, oracle, monkeypatch, tpb, fmt):
+    # the two kernels over both block forms and their sizes, in launches that are
+    # not split (as the choice between them has it): equal bits, within the
+    # short-row bars; without the choice this batch runs as splits
+    heads, kv_heads, dim = 8, 2, 64
+    specs = [(1100, 900, 200), (300, 0, 300), (20, 3, 17)]
+    say("pipelined prefill over blocks", tpb, fmt)
+    dev, ref, ds, rs, qs = build(device, oracle, heads, kv_heads, dim, specs, seed=170 + tpb, tpb=tpb, q8=fmt == "q8_0")
+    starts = [s for _, s, _ in specs]
+    counts = [r for _, _, r in specs]
+
+    def run():
+        attention.profile_reset()
+        out = attention.prefill_batch(dev, np.concatenate(qs), ds, starts, counts, 0, heads, 4096, precision="bf16")
+        return out, attention.profile_read("paged_prefill_merge")[1]
+
+    attention.profile_enable(True)
+    try:
+        (plain, m0), (pipe, m1) = _every_kernel(monkeypatch, run)
+        split, m2 = run()
+    finally:
+        attention.profile_enable(False)
+    assert (m0, m1, m2) == (0, 0, 1)
+    assert _same_bits(plain, pipe)
+    want = np.concatenate([ref.fused_prompt_attention(q, s, 0, st, c, heads, 4096).reshape(c, -1)
+                           for q, s, st, c in zip(qs, rs, starts, counts)])
+    for got in (pipe, split):
+        ok, err = bf16_ok(got, want, SHORT_ROWS)
+        assert ok, err
+
+
 F32_TILE_SPECS = [(1510, 1000, 500), (300, 0, 300), (70, 67, 3), (1, 0, 1)]
 
 

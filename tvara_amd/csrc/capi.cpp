@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <cstdlib>
 #include <cstring>
 #include <limits>
 #include <memory>
@@ -247,7 +248,8 @@ int tvara_attn_prefill(tvara_kv_cache* cache, const uint64_t* sequences, size_t 
             throw std::invalid_argument("unknown attention precision");
         tvara_amd::PrefillPlan& plan = cache->prefill_plan;
         std::vector<uint64_t> key =
-            plan_key(c, {heads, context, static_cast<uint64_t>(precision)}, sequences, count, start, rows);
+            plan_key(c, {heads, context, static_cast<uint64_t>(precision), std::getenv("TVARA_PREFILL_PIPE") ? 1u : 0u},
+                     sequences, count, start, rows);
         if (key != cache->prefill_key || plan.cache != &c) {
             cache->prefill_key.clear();
             plan.build(&c, sequences, count, heads, context, start, rows, precision);

@@ -715,7 +715,8 @@ void PrefillPlan::bf16_splits(const std::vector<int4>& seqs, int kv_heads, int p
     total *= kv_heads;
     splits = 1;
     split_tiles = longest;
-    if (wgs >= kUnits) return;
+    // a choice of the bf16 kernel (prefill.hip) is one between unsplit launches
+    if (wgs >= kUnits || (precision == 1 && std::getenv("TVARA_PREFILL_PIPE"))) return;
     split_tiles = static_cast<int>(
         std::min<int64_t>(std::max<int64_t>({4, (total + kUnits - 1) / kUnits, (longest + 1023) / 1024}), longest));
     if (3 * split_tiles > 2 * longest && longest - split_tiles < 16) split_tiles = longest;

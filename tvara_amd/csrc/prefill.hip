@@ -883,7 +883,8 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_pipe_kernel(const Prefill
 // 128-key tiles 177 us).
 //
 // Key splits (PrefillPlan::bf16_splits) are the plain kernel's: a workgroup
-// then walks a run of the key tiles and leaves a partial.
+// then walks a run of the key tiles and leaves a partial.  A plan made while the
+// variable is set has none; one made without it keeps its splits.
 //
 // x3 (three products per product) always takes the plain kernel, over f32
 // or Q8_0 blocks (d * q dequantised when staged, then split).
