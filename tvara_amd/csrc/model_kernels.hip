@@ -1016,6 +1016,7 @@ __global__ __launch_bounds__(512, 2) void batch_q8_pipe_kernel(const Q8BatchArgs
     };
     load_w(0, ra, da);
     load_x(0, x0);
+    __builtin_amdgcn_sched_barrier(0);  // the first step's wait counts on pair 0 being requested first
     load_w(min(1, np - 1), rb2, db);
     load_x(min(1, np - 1), x1);
     stage(ra, w0);
