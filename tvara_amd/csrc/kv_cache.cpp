@@ -729,20 +729,23 @@ void PrefillPlan::bf16_splits(const std::vector<int4>& seqs, int kv_heads, int p
 // ragged batch, left engines idle while others held the long sequences.  So
 // the list holds only workgroups with rows, in runs of equal work per XCD that
 // keep a (sequence, KV head)'s tiles together, as they share its keys in the
-// XCD's L2, and each XCD's run is ordered from the most keys to the fewest, then
-// from the most rows to the fewest (full and nearly empty chunk tiles by turns
-// would give some engines all the full ones)
-// (MI355X, four chunks of 200-900 tokens after 500-3,000 at head_dim 128 on
-// the three-product tiles: 439 -> 261 us; even batches unchanged).
+// XCD's L2, and each XCD's run is ordered from the most keys to the fewest
+// (MI355X, four chunks of 200-900 tokens after 500-3,000 at head_dim 128 on the
+// three-product tiles: 439 -> 261 us; 8 x (2,048 + 512) unchanged), then from the
+// most rows to the fewest (full and nearly empty chunk tiles by turns gave some
+// engines all the full ones: 64 sequences of 100 tokens after 500 at 9 x 3 heads
+// of 64 41.9 -> 36.2 us; key splits, whose runs are as long by design, stay in
+// their sequences' order).
 //
 // A row's runs follow from its own chunk tile, and only rows of several leave
 // partials, each in its own slots: one long sequence beside many short ones
 // (16 rows after 16,000 tokens beside seven prompts of 512, 32 x 8 heads of 64
 // in f32) takes 4 MB of partials and 163 us, where a slot per row and run of the
 // longest took 854 MB and 425 us (row by row through the decode kernels 291 us);
-// with heads of 128 8 MB and 302 us, 1,678 MB and 855 us (518 us).  prefill_f32_shape and bf16_splits aim at 1,024 and 256 runs
-// of work, so a plan has at most twice that many workgroups with partials, of
-// 128 and 256 (row, head) pairs: 136 MB at head_dim 128.
+// with heads of 128 8 MB and 302 us, 1,678 MB and 855 us (518 us).
+// prefill_f32_shape and bf16_splits aim at 1,024 and 256 runs of work, so a plan
+// has at most twice that many workgroups with partials, of 128 and 256 (row,
+// head) pairs: 136 MB at head_dim 128.
 std::vector<int4> PrefillPlan::work_list(const std::vector<int4>& seqs, int kv_heads, int positions,
                                          std::vector<int2>& row_runs) {
     constexpr int kXcds = 8, kCus = 32, kTileKeys = 64;
@@ -789,9 +792,9 @@ std::vector<int4> PrefillPlan::work_list(const std::vector<int4>& seqs, int kv_h
         before += items[i].end - items[i].tile0;
     }
     for (auto& r : run)
-        std::stable_sort(r.begin(), r.end(), [](const Item& a, const Item& b) {
+        std::stable_sort(r.begin(), r.end(), [this](const Item& a, const Item& b) {
             const int ta = a.end - a.tile0, tb = b.end - b.tile0;
-            return ta != tb ? ta > tb : a.rows > b.rows;
+            return ta != tb ? ta > tb : splits == 1 && a.rows > b.rows;
         });
     size_t longest = 0;
     for (const auto& r : run) longest = std::max(longest, r.size());

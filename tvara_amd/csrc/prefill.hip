@@ -491,6 +491,8 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_bf16_kernel(const Prefill
     }
 
     bool bad = false;
+    // the workgroup's first row's (its rows have as many runs, in slots that follow)
+    const int2 runs = a.row_runs ? a.row_runs[sd.w + q0] : make_int2(0, 1);
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
         // row 0 of the normaliser tile: lane r16 (group 0), element 0
@@ -500,9 +502,8 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_bf16_kernel(const Prefill
         size_t at = static_cast<size_t>(sd.w + pos) * a.heads + head;
         float* o = a.out + at * D + 4 * g;
         float div = l;
-        const int2 runs = a.row_runs ? a.row_runs[sd.w + pos] : make_int2(0, 1);
         if (runs.y > 1) {  // a partial
-            at = static_cast<size_t>(runs.x + (wk.x >> 16)) * a.heads + head;
+            at = static_cast<size_t>(runs.x + (pos - q0) * runs.y + (wk.x >> 16)) * a.heads + head;
             if (g == 0) *reinterpret_cast<float2*>(a.part_ml + 2 * at) = make_float2(m[nt], l);
             o = a.part_acc + at * D + 4 * g;
             bad |= !__builtin_isfinite(l);

@@ -321,6 +321,8 @@ __global__ __launch_bounds__(64 * kRowsPerGroup / (16 * NT), 2) void prefill_f32
     }
 
     if (__any(nonfinite != 0.f) && lane == 0) *a.err = 1;
+    // the workgroup's first row's (its rows have as many runs, in slots that follow)
+    const int2 runs = a.row_runs ? a.row_runs[sd.w + q0] : make_int2(0, 1);
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
         const float total = cross_row_sum(l[nt]);
@@ -329,9 +331,8 @@ __global__ __launch_bounds__(64 * kRowsPerGroup / (16 * NT), 2) void prefill_f32
         size_t at = static_cast<size_t>(sd.w + pos[nt]) * a.heads + head[nt];
         float* o = a.out + at * D + 16 * g;
         float inv = total;
-        const int2 runs = a.row_runs ? a.row_runs[sd.w + pos[nt]] : make_int2(0, 1);
         if (runs.y > 1) {
-            at = static_cast<size_t>(runs.x + split) * a.heads + head[nt];
+            at = static_cast<size_t>(runs.x + (pos[nt] - q0) * runs.y + split) * a.heads + head[nt];
             if (g == 0) *reinterpret_cast<float2*>(a.part_ml + 2 * at) = make_float2(m[nt], total);
             if (m[nt] == -INFINITY) continue;  // no key of this run: not used either
             o = a.part_acc + at * D + 16 * g;
