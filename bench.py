@@ -466,9 +466,9 @@ def bench_prefill(args, w, precision="bf16"):
     steps = args.steps if precision != "f32" else max(1, min(args.steps, 20))
     ms_per_step = timed_steps(call, steps)
     kernel = {"bf16": "paged_prefill_bf16", "f32x3": "paged_prefill_x3", "f32": "paged_prefill_f32"}[precision]
-    kt = kernel_times(call, steps, [kernel, "paged_decode_merge"])
+    kt = kernel_times(call, steps, [kernel, "paged_prefill_merge"])
     kernel_ms, _ = kt[kernel]
-    merge_ms, merges = kt["paged_decode_merge"]
+    merge_ms, merges = kt["paged_prefill_merge"]
     plan.check()
     assert np.isfinite(out.numpy()).all()
     tfs = w.flops() / (kernel_ms * 1e-3) / 1e12
