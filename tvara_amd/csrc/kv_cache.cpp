@@ -700,7 +700,10 @@ void AttnPlan::check_after(hipEvent_t after) {
 // of 200-260 tiles: 547 us against 770 in 512 units and 602 in 1,024), and so
 // does one that shortens the longest walk by less than a third and 16 tiles: 64
 // sequences of 40 tokens after 500 at 9 x 3 heads of 64, 192 workgroups of nine
-// tiles, 17 us against 27 in runs of seven and two.
+// tiles, 17 us against 27 in runs of seven and two.  Nor is the merge worth less
+// than six tiles (four of three products): a fresh chunk of 512 tokens at 32 x 8
+// heads of 64, runs of four of its eight tiles, 17.4 us against 17.6 (23.9
+// against 27.4), while the plan allocates its partials.
 void PrefillPlan::bf16_splits(const std::vector<int4>& seqs, int kv_heads, int positions) {
     constexpr int64_t kUnits = 256;
     int64_t wgs = 0, total = 0;
@@ -719,7 +722,8 @@ void PrefillPlan::bf16_splits(const std::vector<int4>& seqs, int kv_heads, int p
     if (wgs >= kUnits || (precision == 1 && std::getenv("TVARA_PREFILL_PIPE"))) return;
     split_tiles = static_cast<int>(
         std::min<int64_t>(std::max<int64_t>({4, (total + kUnits - 1) / kUnits, (longest + 1023) / 1024}), longest));
-    if (3 * split_tiles > 2 * longest && longest - split_tiles < 16) split_tiles = longest;
+    const int saved = longest - split_tiles;
+    if (saved < (precision == 1 ? 6 : 4) || (3 * split_tiles > 2 * longest && saved < 16)) split_tiles = longest;
     splits = (longest + split_tiles - 1) / split_tiles;
 }
 
